@@ -1491,7 +1491,7 @@ int enqueue_device_step(cohx_ctx *ctx, Workspace &w, const Prepared &p, int kv_g
       launch_qkv_post(s, R, sd, w.qkv, ly.bqkv, ctx->rope, w.row_pos, w.row_slot, w.q_rot, kp, vp,
                       w.row_err);
       prof_end(ctx, e);
-    } else if (ly.qkv.view.dtype != kFmtQ8 && ly.qkv.view.dtype != kFmtQ4) {
+    } else if (ly.qkv.view.dtype == kFmtKQ || (f16_gemm && ly.qkv.view.dtype == kFmtF16)) {
       e = prof_begin(ctx, kCatMvQkv, matrix_pass_bytes(ly.qkv, R, H + 2 * KVD, false),
                      2.0 * R * (H + 2 * KVD) * H);
       launch_matvec(s, kEpiStore, ly.qkv.view, act, R,
@@ -1502,9 +1502,9 @@ int enqueue_device_step(cohx_ctx *ctx, Workspace &w, const Prepared &p, int kv_g
                       w.row_err);
       prof_end(ctx, e);
     } else {
-      // Q8_0/Q4_0: bias, RoPE and the K/V append run in the matvec's epilogue
-      // (rows uploaded in rope_row order); the bytes are the matrix pass plus
-      // the post pass's writes
+      // Q8_0/Q4_0 and exact F16: bias, RoPE and the K/V append run in the
+      // matvec's epilogue (Q8_0/Q4_0 rows uploaded in rope_row order); the
+      // bytes are the matrix pass plus the post pass's writes
       e = prof_begin(ctx, kCatMvQkv, b_qkv_fused, 2.0 * R * (H + 2 * KVD) * H);
       launch_matvec_qkv(s, ly.qkv.view, act, R, MatvecOut{nullptr, 0, nullptr, nullptr, w.row_err, nullptr}, qe);
       prof_end(ctx, e);
@@ -1603,8 +1603,7 @@ int enqueue_device_step(cohx_ctx *ctx, Workspace &w, const Prepared &p, int kv_g
       prof_end(ctx, e);
     }
     if (!fused_quant && a_down == kActF16) {
-      // F16 in the packed-prefill regime: gate+up on the matrix cores with
-      // SwiGLU in the epilogue, writing the down projection's binary16
+      // F16: gate+up with SwiGLU in the epilogue, writing the down projection's binary16
       // operand into the f32 SwiGLU rows' space, w.h (act.f16 holds gate+up's
       // own operand, which other workgroups are still reading); false:
       // nothing launched

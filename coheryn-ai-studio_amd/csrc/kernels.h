@@ -121,12 +121,11 @@ bool launch_matvec(hipStream_t s, Epilogue epi, const MatrixView &w, const ActVi
 // to even.
 bool launch_matvec_swiglu_q8(hipStream_t s, const MatrixView &w, const ActView &act, int rows_b,
                              const MatvecOut &o, const ActView &qout, int qout_nbp);
-// F16 gate+up of a step in the packed-prefill regime on the matrix-core GEMM
-// (gemm.h) with SwiGLU in its epilogue, writing the down projection's
-// binary16 operand rows out_f16[rows_b][F] directly (the rounding and
-// non-finite checks of launch_quant_act(kActF16)).  Returns false (nothing
-// launched) outside the regime (set_prefill_mfma off, under 128 rows, not
-// F16) or when K is not a multiple of 64.
+// F16 gate+up with SwiGLU in its epilogue (the regime's GEMM, gemm.h, in a
+// step of the packed-prefill regime, else the exact f64 kernels), writing the
+// down projection's binary16 operand rows out_f16[rows_b][F] directly (the
+// rounding and non-finite checks of launch_quant_act(kActF16)).  Returns false
+// (nothing launched) for other formats or when K is not a multiple of 32.
 bool launch_matvec_swiglu_f16(hipStream_t s, const MatrixView &w, const ActView &act, int rows_b,
                               const MatvecOut &o, uint16_t *out_f16);
 // Q8_0/Q4_0 linears of a step in the packed-prefill regime on the matrix
@@ -153,10 +152,10 @@ struct QkvEpi {
   float *kpool, *vpool;      // the layer's pools
   int H, KVD, D, NKV;
 };
-// Q8_0/Q4_0 qkv projection with launch_qkv_post's work in its epilogue, for
-// weights whose query and key rows were uploaded in rope_row order.  Gives
-// the same bits as the matvec and launch_qkv_post in sequence; out.out is
-// unused.
+// Exact qkv projection with launch_qkv_post's work in its epilogue: Q8_0/Q4_0
+// weights whose query and key rows were uploaded in rope_row order, F16 rows
+// in the source order (K and D multiples of 32).  Gives the same bits as the
+// matvec and launch_qkv_post in sequence; out.out is unused.
 void launch_matvec_qkv(hipStream_t s, const MatrixView &w, const ActView &act, int rows_b,
                        const MatvecOut &o, const QkvEpi &q);
 // The packed-prefill regime's qkv projection with the same work in the

@@ -14,6 +14,10 @@
 #include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
+#include <cstdio>
+#include <cstdlib>
+#include <type_traits>
+
 #include "device.h"
 #include "gemm.h"
 #include "kernels.h"
@@ -1573,191 +1577,331 @@ __global__ __launch_bounds__(256) void k_argmax_reduce(const unsigned long long 
 }
 
 // ---------------------------------------------------------------------------
-// F16 matvec with the reference's wide reduction (cpu.rs:31-35 over
-// round_f16 operands): f32 products of binary16 values are exact, summed in
-// f64 per lane in element order, then across lanes in a fixed butterfly.
-// One wave per output row; kEpiSwiglu pairs row i with row i + F.
+// F16 matvec for any width (cpu.rs:31-35 over round_f16 operands; K not a
+// multiple of 32, which no model matrix is): f32 products of binary16 values
+// are exact, summed in f64 per lane in element order, then across lanes in a
+// fixed butterfly.  One wave per output row.
 // ---------------------------------------------------------------------------
-template <int kEpi>
 __global__ __launch_bounds__(256) void k_mv_f16(MatrixView w, ActView act, int rows_b,
                                                 MatvecOut o) {
   const int lane = threadIdx.x % kWave;
   const int row = blockIdx.x * 4 + threadIdx.x / kWave;
-  const int out_rows = kEpi == kEpiSwiglu ? w.rows / 2 : w.rows;
-  if (row >= out_rows) return;
+  if (row >= w.rows) return;
   const int K = w.K;
   const uint16_t *wr = w.f16 + (size_t)row * K;
-  const uint16_t *wu = kEpi == kEpiSwiglu ? w.f16 + (size_t)(row + out_rows) * K : nullptr;
   for (int r = 0; r < rows_b; r++) {
     const uint16_t *ar = act.f16 + (size_t)r * K;
-    double s = -0.0, su = -0.0;
-    for (int k = lane; k < K; k += kWave) {
-      const float a = h2f(ar[k]);
-      s += (double)(h2f(wr[k]) * a);
-      if (kEpi == kEpiSwiglu) su += (double)(h2f(wu[k]) * a);
-    }
-    s = wave_sum_f64(s);
-    if (kEpi == kEpiSwiglu) su = wave_sum_f64(su);
-    const float v = (float)s;
-    const int er = o.err_rows ? (int)o.err_rows[r] : r;
-    if (kEpi == kEpiArgmax) {
-      if (o.logits && lane == 0) o.logits[(size_t)r * w.rows + row] = v;
-      if (lane == 0) {
-        if (!finitef(v)) atomicOr(&o.row_err[er], kErrNonFinite);
-        atomicMax(o.argmax + r, argmax_key(v, row));
-      }
-    } else if (kEpi == kEpiSwiglu) {
-      const float u = (float)su;
-      if (lane == 0) {
-        if (!finitef(v) || !finitef(u)) atomicOr(&o.row_err[er], kErrNonFinite);
-        o.out[(size_t)r * o.ld + row] = (v / (1.0f + exp_f32(-v))) * u;
-      }
-    } else if (lane == 0) {
-      if (!finitef(v)) atomicOr(&o.row_err[er], kErrNonFinite);
-      float *p = o.out + (size_t)r * o.ld + row;
-      if (kEpi == kEpiResidual)
-        *p = *p + v;
-      else
-        *p = v;
+    double s = -0.0;
+    for (int k = lane; k < K; k += kWave) s += (double)(h2f(wr[k]) * h2f(ar[k]));
+    const float v = (float)wave_sum_f64(s);
+    if (lane == 0) {
+      if (!finitef(v)) atomicOr(&o.row_err[o.err_rows ? (int)o.err_rows[r] : r], kErrNonFinite);
+      o.out[(size_t)r * o.ld + row] = v;
     }
   }
 }
 
 // ---------------------------------------------------------------------------
-// F16 matvec for batches of 16..127 rows, in the reference's exact order: lane
-// = batch row, each dot one sequential f64 chain over k from -0.0
-// (cpu.rs:31-35 over round_f16 operands), f32 result.  A wave owns 4 output
-// rows (4 gate + 4 up rows for SwiGLU) and one pass of up to 64 batch rows;
-// the weight rows are wave-uniform loads, the activation rows per lane.  The
-// argmax epilogue leaves one key per (batch row, 16-row tile) for
-// k_argmax_reduce.
+// F16 matvec on the f64 matrix cores (cpu.rs:31-35 over round_f16 operands).
+// The product of two binary16 values is exact in f32 and in f64, so
+// v_mfma_f64_16x16x4 sums exactly the terms of the reference's f64 dot, each
+// addition rounded once (the instruction is a chain of four fma).  Every such
+// product is a multiple of 2^-48: a dot whose partial sums stay below 2^5 is
+// exact in f64 in any order, and a larger one rounds at 2^-53 of its size
+// before its final rounding to f32.  The order here is fixed: wave w of the
+// workgroup takes the 32-input blocks w, w + kW, ...; within a block lane
+// group g holds inputs 8g .. 8g+7 (one 16-byte load) and step e multiplies
+// input 8g + e of every group; the waves' sums are added in wave order.
+//
+// A workgroup owns kNM tiles of 16 output rows x kNN tiles of 16 batch rows.
+// Lane l of an operand tile brings row l % 16 (weights and activations are
+// row-major, so a wave's load of a tile is 16 rows x 64 bytes), the loads run
+// two blocks ahead of their use.  What bounds it is the f64 matrix rate: 31 ns
+// per instruction and SIMD (1,024 products), against about 75 ns for the same
+// products as f32 multiply, widening and f64 add on the vector unit.
+// kEpiSwiglu pairs gate tile u with up tile u (row + F), kEpiQkv the two tiles
+// that hold the RoPE halves of the same 16 head elements.
+//   Measured at 56 rows (Qwen2.5-0.5B shape), against one f64 chain per lane
+// on the vector unit: o 5.7 and down 16.4 us (145 the two on average before),
+// gate+up 25 (168 and a rounding pass of 4.7), qkv with its bias, RoPE and K/V
+// append 8.5 (46.7 and 4.8), head 324 (1,184).
 // ---------------------------------------------------------------------------
-template <int kEpi>
-__global__ __launch_bounds__(256) void k_mv_f16s(MatrixView w, ActView act, int rows_b,
-                                                 MatvecOut o) {
-  constexpr int kQ = kEpi == kEpiSwiglu ? 8 : 4;
-  __shared__ unsigned long long s_key[4][kWave];
-  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
-  const int out_rows = kEpi == kEpiSwiglu ? w.rows / 2 : w.rows;
-  const int o0 = (blockIdx.x * 4 + wave) * 4;
-  const int r = blockIdx.y * kWave + lane;
-  const int K = w.K;
-  const int rr = min(r, rows_b - 1);
-  const uint16_t *xr = act.f16 + (size_t)rr * K;
-  const uint16_t *wq[kQ];
-#pragma unroll
-  for (int q = 0; q < kQ; q++) {
-    int row = o0 + (q % 4);
-    row = min(row, out_rows - 1);
-    if (kEpi == kEpiSwiglu && q >= 4) row += out_rows;
-    wq[q] = w.f16 + (size_t)row * K;
-  }
-  double acc[kQ];
-#pragma unroll
-  for (int q = 0; q < kQ; q++) acc[q] = -0.0;
-  for (int k0 = 0; k0 < K; k0 += 8) {
-    const uint4 xv = *reinterpret_cast<const uint4 *>(xr + k0);
-    const uint32_t xw[4] = {xv.x, xv.y, xv.z, xv.w};
-    uint4 wv[kQ];
-#pragma unroll
-    for (int q = 0; q < kQ; q++) wv[q] = *reinterpret_cast<const uint4 *>(wq[q] + k0);
-#pragma unroll
-    for (int e = 0; e < 8; e++) {
-      const float a = h2f((uint16_t)(xw[e / 2] >> (16 * (e % 2))));
-#pragma unroll
-      for (int q = 0; q < kQ; q++) {
-        const uint32_t ww[4] = {wv[q].x, wv[q].y, wv[q].z, wv[q].w};
-        acc[q] += (double)(h2f((uint16_t)(ww[e / 2] >> (16 * (e % 2)))) * a);
-      }
-    }
-  }
-  const bool rvalid = r < rows_b;
-  const int er = (rvalid && o.err_rows) ? (int)o.err_rows[r] : r;
+typedef double v4d __attribute__((ext_vector_type(4)));
+
+// One output of the F16 kernels below: v[0] is row orow of batch row r (v[1]
+// its pair: the up row, or element i + D/2 of the head).  kEpiArgmax: 16
+// consecutive lanes hold the 16 rows of tile `tile` (`row` is the place in it).
+template <int kEpi, int kNM>
+__device__ __forceinline__ void f16_epilogue(const float (&v)[kNM], bool rvalid, int r, int orow, int row,
+                                             const MatrixView &w, const MatvecOut &o, const QkvEpi &qe,
+                                             uint16_t *out16, int tiles, int tile) {
   bool bad = false;
-  if (kEpi == kEpiArgmax) {
-    unsigned long long best = 0ull;
+  const int F = w.rows / 2;
+      if constexpr (kEpi == kEpiArgmax) {
+        const bool valid = rvalid && orow < w.rows;
+        if (valid) {
+          bad = !finitef(v[0]);
+          if (o.logits) o.logits[(size_t)r * w.rows + orow] = v[0];
+        }
+        unsigned long long key = valid ? argmax_key(v[0], orow) : 0ull;
 #pragma unroll
-    for (int q = 0; q < 4; q++) {
-      const int row = o0 + q;
-      if (!rvalid || row >= w.rows) continue;
-      const float v = (float)acc[q];
-      bad |= !finitef(v);
-      if (o.logits) o.logits[(size_t)r * w.rows + row] = v;
-      const unsigned long long key = argmax_key(v, row);
-      best = key > best ? key : best;
-    }
-    s_key[wave][lane] = best;
-    __syncthreads();
-    if (wave == 0 && rvalid) {
-      unsigned long long b = s_key[0][lane];
+        for (int s = 1; s < 16; s <<= 1) {
+          const unsigned long long x = __shfl_xor(key, s, kWave);
+          key = x > key ? x : key;
+        }
+        if (rvalid && row == 0) o.argmax[(size_t)r * tiles + tile] = key;
+      } else if constexpr (kEpi == kEpiQkv) {
+        // k_qkv_post's arithmetic: element i of a head in v[0], i + D/2 in v[1]
+        if (rvalid) {
+          bad = !finitef(v[0]) || !finitef(v[kNM - 1]);
+          const uint32_t pos = qe.row_pos[r];
+          const int32_t slot = qe.row_slot[r];
+          const int half = qe.D / 2, page = slot / kPage, off = slot % kPage;
+          const int head = orow / qe.D, i = orow % qe.D;
+          const float a = v[0] + qe.bias[orow], b = v[kNM - 1] + qe.bias[orow + half];
+          const int nh = qe.H / qe.D;
+          if (head < nh + qe.NKV) {
+            const float2 cs = qe.rope[(size_t)pos * half + i];
+            const float ya = fmaf(a, cs.x, -(b * cs.y)), yb = fmaf(a, cs.y, b * cs.x);
+            if (head < nh) {
+              float *q = qe.q_rot + (size_t)r * qe.H + orow;
+              q[0] = ya;
+              q[half] = yb;
+            } else if (slot >= 0) {
+              qe.kpool[k_at(page, pos / kPage, head - nh, qe.NKV, off, i, qe.D)] = ya;
+              qe.kpool[k_at(page, pos / kPage, head - nh, qe.NKV, off, i + half, qe.D)] = yb;
+            }
+          } else if (slot >= 0) {
+            qe.vpool[v_at(page, head - nh - qe.NKV, qe.NKV, off, i, qe.D)] = a;
+            qe.vpool[v_at(page, head - nh - qe.NKV, qe.NKV, off, i + half, qe.D)] = b;
+          }
+        }
+      } else if (rvalid) {
+        if constexpr (kEpi == kEpiSwiglu) {
+          if (orow < F) {
+            const float g = v[0], u = v[kNM - 1];
+            bad = !finitef(g) || !finitef(u);
+            const float y = (g / (1.0f + exp_f32(-g))) * u;
+            if (out16) {  // k_quant_act<1>'s rounding and check
+              const uint16_t h = f2h(y);
+              bad |= !finitef(h2f(h));
+              out16[(size_t)r * F + orow] = h;
+            } else {
+              o.out[(size_t)r * o.ld + orow] = y;
+            }
+          }
+        } else if (orow < w.rows) {
+          bad = !finitef(v[0]);
+          float *p = o.out + (size_t)r * o.ld + orow;
+          *p = kEpi == kEpiResidual ? *p + v[0] : v[0];
+        }
+      }
+  if (bad) atomicOr(&o.row_err[o.err_rows ? (int)o.err_rows[r] : r], kErrNonFinite);
+}
+
+template <int kEpi, int kNM, int kNN, int kW>
+__global__ __launch_bounds__(64 * kW) void k_mv_f16m(MatrixView w, ActView act, int rows_b, int n_tiles,
+                                                     MatvecOut o, QkvEpi qe, uint16_t *out16) {
+  static_assert(kNM == (kEpi == kEpiSwiglu || kEpi == kEpiQkv ? 2 : 1), "paired tiles");
+  constexpr int kLd = 17;  // padded column of a parked tile: conflict-free both ways
+  extern __shared__ double s_part[];  // [kW][kNM * kNN][16 * kLd]
+  const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int F = w.rows / 2, hp = kEpi == kEpiQkv ? qe.D / 32 : 1;  // hp: tile pairs per head
+  const int units = kEpi == kEpiSwiglu ? (F + 15) / 16 : kEpi == kEpiQkv ? w.rows / 32 : w.mtiles;
+  // all batch groups of a unit on one XCD (blockIdx % 8): its weights enter that L2 once
+  const int ngroups = (n_tiles + kNN - 1) / kNN;
+  const int ug = blockIdx.x / (8 * ngroups), rem = blockIdx.x % (8 * ngroups);
+  const int ng = rem / 8, unit = ug * 8 + rem % 8;
+  if (unit >= units) return;
+  const int K = w.K, nb = K / 32;
+  const int r16 = lane % 16, koff = 8 * (lane / 16);
+  int row0[kNM];  // first output row of each tile
+  if constexpr (kEpi == kEpiQkv) {
+    row0[0] = unit / hp * qe.D + unit % hp * 16;
+    row0[kNM - 1] = row0[0] + qe.D / 2;
+  } else {
+    row0[0] = unit * 16;
+    if constexpr (kEpi == kEpiSwiglu) row0[kNM - 1] = F + unit * 16;
+  }
+  const uint16_t *wp[kNM], *xp[kNN];
 #pragma unroll
-      for (int i = 1; i < 4; i++) b = s_key[i][lane] > b ? s_key[i][lane] : b;
-      o.argmax[(size_t)r * w.mtiles + blockIdx.x] = b;
-    }
-  } else if (rvalid) {
+  for (int m = 0; m < kNM; m++) {  // rows past the matrix repeat its last row
+    const int last = kEpi == kEpiSwiglu && m == 0 ? F - 1 : w.rows - 1;
+    wp[m] = w.f16 + (size_t)min(row0[m] + r16, last) * K + koff;
+  }
 #pragma unroll
-    for (int q = 0; q < 4; q++) {
-      const int row = o0 + q;
-      if (row >= out_rows) continue;
-      float v = (float)acc[q];
-      float *p = o.out + (size_t)r * o.ld + row;
-      if (kEpi == kEpiSwiglu) {
-        const float u = (float)acc[q + 4];
-        bad |= !finitef(v) || !finitef(u);
-        *p = (v / (1.0f + exp_f32(-v))) * u;
-      } else {
-        bad |= !finitef(v);
-        *p = kEpi == kEpiResidual ? *p + v : v;
+  for (int n = 0; n < kNN; n++)  // rows past the batch repeat its last row
+    xp[n] = act.f16 + (size_t)min((ng * kNN + n) * 16 + r16, rows_b - 1) * K + koff;
+  v4d acc[kNM][kNN];
+#pragma unroll
+  for (int m = 0; m < kNM; m++)
+#pragma unroll
+    for (int n = 0; n < kNN; n++) acc[m][n] = v4d{-0.0, -0.0, -0.0, -0.0};
+  struct Block {
+    u32x4v a[kNM], b[kNN];
+  };
+  auto load = [&](Block &blk, int t) {  // past the end: the last block again, unused
+    const int k = 32 * min(t, nb - 1);
+#pragma unroll
+    for (int m = 0; m < kNM; m++) blk.a[m] = *reinterpret_cast<const u32x4v *>(wp[m] + k);
+#pragma unroll
+    for (int n = 0; n < kNN; n++) blk.b[n] = *reinterpret_cast<const u32x4v *>(xp[n] + k);
+  };
+  constexpr int kD = 3;
+  Block ring[kD];
+#pragma unroll
+  for (int i = 0; i < kD - 1; i++) load(ring[i], wave + i * kW);
+  for (int t0 = wave; t0 < nb; t0 += kD * kW) {
+#pragma unroll
+    for (int u = 0; u < kD; u++) {
+      const int t = t0 + u * kW;
+      load(ring[(u + kD - 1) % kD], t + (kD - 1) * kW);
+      if (t < nb) {
+        const Block &blk = ring[u];
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+          double a[kNM];
+#pragma unroll
+          for (int m = 0; m < kNM; m++) a[m] = (double)h2f((uint16_t)(blk.a[m][e / 2] >> (16 * (e % 2))));
+#pragma unroll
+          for (int n = 0; n < kNN; n++) {
+            const double b = (double)h2f((uint16_t)(blk.b[n][e / 2] >> (16 * (e % 2))));
+#pragma unroll
+            for (int m = 0; m < kNM; m++)
+              acc[m][n] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[m], b, acc[m][n], 0, 0, 0);
+          }
+        }
       }
     }
   }
-  if (bad) atomicOr(&o.row_err[er], kErrNonFinite);
+  // D layout: lane l, slot i: output row l / 16 + 4 i, batch row l % 16
+#pragma unroll
+  for (int m = 0; m < kNM; m++)
+#pragma unroll
+    for (int n = 0; n < kNN; n++)
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+        s_part[(size_t)((wave * kNM + m) * kNN + n) * (16 * kLd) + r16 * kLd + lane / 16 + 4 * i] = acc[m][n][i];
+  __syncthreads();
+  // ---- epilogue: thread -> (batch row, output row); 16 consecutive threads
+  // hold the 16 outputs of one batch row
+  for (int idx = threadIdx.x; idx < kNN * 256; idx += 64 * kW) {
+    const int n = idx / 256, col = idx % 256 / 16, row = idx % 16;
+    const int r = (ng * kNN + n) * 16 + col;
+    const bool rvalid = r < rows_b;
+    float v[kNM];
+#pragma unroll
+    for (int m = 0; m < kNM; m++) {
+      double sum = s_part[(size_t)(m * kNN + n) * (16 * kLd) + col * kLd + row];
+#pragma unroll
+      for (int i = 1; i < kW; i++) sum += s_part[(size_t)((i * kNM + m) * kNN + n) * (16 * kLd) + col * kLd + row];
+      v[m] = (float)sum;
+    }
+    f16_epilogue<kEpi, kNM>(v, rvalid, r, row0[0] + row, row, w, o, qe, out16, units, unit);
+  }
 }
 
 // ---------------------------------------------------------------------------
-// F16 LM head with argmax: the same per-output arithmetic as k_mv_f16 (f64
-// per lane in element order, fixed butterfly), 16 vocabulary rows per
-// workgroup (4 per wave); each batch row's best key over the 16 rows goes to
-// part[r][tile] for k_argmax_reduce, so no output contends on an atomic.
+// The same product for batches of up to 16 rows on v_mfma_f64_4x4x4 (four
+// blocks of 4 x 4 x 4): a wave owns 4 output rows x 4 kNN batch rows and its
+// four blocks are four groups of inputs, so a matrix of 896 rows gives 224
+// units instead of 56, a few batch rows cost a quarter of a 16 x 16 tile, and
+// a wave's load of its weights is 4 rows x 256 contiguous bytes.  Lane l holds
+// row l % 4 and inputs 8 (l / 4) .. + 7 of each 128-input chunk (block l / 4 %
+// 4, k index l / 16 of the instruction).  A workgroup is kQ quads of rows x kS
+// waves that split the chunks of K; the blocks' and waves' sums meet in LDS
+// in a fixed order.  The head takes kQ = 4, kS = 1 (whole 16-row tiles).
+//   8.7 ns per instruction and SIMD for 256 products (20 ns when it depends
+// on the one before).  Measured at 4 rows, against one wave per output and one
+// row after the other: o 3.9 and down 5.9 us (53 on average before), gate+up
+// 7.5 (22.4 and a rounding pass of 4.6), qkv 5.5 (17.8 and 4.7), head 67 for
+// its 272 MB (532).
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_head_f16(MatrixView w, ActView act, int rows_b,
-                                                  MatvecOut o) {
-  __shared__ unsigned long long s_key[4];
-  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
-  const int row0 = blockIdx.x * 16 + wave * 4;
-  const int K = w.K, units = w.mtiles;
-  for (int r = 0; r < rows_b; r++) {
-    const uint16_t *ar = act.f16 + (size_t)r * K;
-    double acc[4] = {-0.0, -0.0, -0.0, -0.0};
-    for (int k = lane; k < K; k += kWave) {
-      const float a = h2f(ar[k]);
+template <int kEpi, int kNM, int kNN, int kQ, int kS>
+__global__ __launch_bounds__(64 * kQ * kS) void k_mv_f16v(MatrixView w, ActView act, int rows_b, MatvecOut o,
+                                                          QkvEpi qe, uint16_t *out16) {
+  static_assert(kNM == (kEpi == kEpiSwiglu || kEpi == kEpiQkv ? 2 : 1), "paired quads");
+  static_assert(kEpi != kEpiArgmax || (kQ == 4 && kS == 1), "the head's keys are per 16-row tile");
+  __shared__ double s_part[kQ * kS][kNM * kNN][64];
+  const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int quad = wave / kS, split = wave % kS;
+  const int F = w.rows / 2, K = w.K, nc = (K + 127) / 128;
+  const int hq = kEpi == kEpiQkv ? qe.D / 8 : 1;  // quad pairs per head
+  auto first = [&](int u) { return kEpi == kEpiQkv ? u / hq * qe.D + u % hq * 4 : u * 4; };
+  const int row0 = first(blockIdx.x * kQ + quad), pair = kEpi == kEpiQkv ? qe.D / 2 : F;
+  const int limit = kEpi == kEpiSwiglu ? F : w.rows;
+  const int koff = 8 * (lane / 4);
+  const uint16_t *wp[kNM], *xp[kNN];
 #pragma unroll
-      for (int q = 0; q < 4; q++)
-        if (row0 + q < w.rows) acc[q] += (double)(h2f(w.f16[(size_t)(row0 + q) * K + k]) * a);
-    }
-    const int er = o.err_rows ? (int)o.err_rows[r] : r;
-    unsigned long long best = 0ull;
-    bool bad = false;
+  for (int m = 0; m < kNM; m++)  // rows past the matrix repeat its last row
+    wp[m] = w.f16 + (size_t)(min(row0 + lane % 4, (kEpi == kEpiQkv ? limit - pair : limit) - 1) + m * pair) * K;
 #pragma unroll
-    for (int q = 0; q < 4; q++) {
-      const float v = (float)wave_sum_f64(acc[q]);
-      const int row = row0 + q;
-      if (row >= w.rows) continue;
-      bad |= !finitef(v);
-      if (o.logits && lane == 0) o.logits[(size_t)r * w.rows + row] = v;
-      const unsigned long long key = argmax_key(v, row);
-      best = key > best ? key : best;
-    }
-    if (bad && lane == 0) atomicOr(&o.row_err[er], kErrNonFinite);
-    if (lane == 0) s_key[wave] = best;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      unsigned long long b = s_key[0];
+  for (int n = 0; n < kNN; n++) xp[n] = act.f16 + (size_t)min(n * 4 + lane % 4, rows_b - 1) * K;
+  double acc[kNM][kNN];
 #pragma unroll
-      for (int i = 1; i < 4; i++) b = s_key[i] > b ? s_key[i] : b;
-      o.argmax[(size_t)r * units + blockIdx.x] = b;
+  for (int m = 0; m < kNM; m++)
+#pragma unroll
+    for (int n = 0; n < kNN; n++) acc[m][n] = -0.0;
+  struct Chunk {
+    u32x4v a[kNM], b[kNN];
+  };
+  const u32x4v none = {0u, 0u, 0u, 0u};
+  auto load = [&](Chunk &c, int t) {  // inputs past K: zero products
+    const int k = 128 * t + koff;
+    const bool in = k < K;
+#pragma unroll
+    for (int m = 0; m < kNM; m++) c.a[m] = in ? *reinterpret_cast<const u32x4v *>(wp[m] + k) : none;
+#pragma unroll
+    for (int n = 0; n < kNN; n++) c.b[n] = in ? *reinterpret_cast<const u32x4v *>(xp[n] + k) : none;
+  };
+  constexpr int kD = 3;
+  Chunk ring[kD];
+#pragma unroll
+  for (int i = 0; i < kD - 1; i++) load(ring[i], split + i * kS);
+  for (int t0 = split; t0 < nc; t0 += kD * kS) {
+#pragma unroll
+    for (int u = 0; u < kD; u++) {
+      const int t = t0 + u * kS;
+      load(ring[(u + kD - 1) % kD], t + (kD - 1) * kS);
+      if (t < nc) {
+        const Chunk &c = ring[u];
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+          double a[kNM];
+#pragma unroll
+          for (int m = 0; m < kNM; m++) a[m] = (double)h2f((uint16_t)(c.a[m][e / 2] >> (16 * (e % 2))));
+#pragma unroll
+          for (int n = 0; n < kNN; n++) {
+            const double b = (double)h2f((uint16_t)(c.b[n][e / 2] >> (16 * (e % 2))));
+#pragma unroll
+            for (int m = 0; m < kNM; m++) acc[m][n] = __builtin_amdgcn_mfma_f64_4x4x4f64(a[m], b, acc[m][n], 0, 0, 0);
+          }
+        }
+      }
     }
-    __syncthreads();
+  }
+  // D layout: lane l: output row l / 16, batch row l % 4, block l / 4 % 4
+#pragma unroll
+  for (int m = 0; m < kNM; m++)
+#pragma unroll
+    for (int n = 0; n < kNN; n++) s_part[wave][m * kNN + n][lane] = acc[m][n];
+  __syncthreads();
+  constexpr int kRows = 4 * kQ;
+  for (int idx = threadIdx.x; idx < kRows * 4 * kNN; idx += 64 * kQ * kS) {
+    const int row = idx % kRows, r = idx / kRows, n = r / 4;
+    const int at = row % 4 * 16 + r % 4;
+    float v[kNM];
+#pragma unroll
+    for (int m = 0; m < kNM; m++) {
+      double sum = -0.0;
+#pragma unroll
+      for (int i = 0; i < kS; i++)
+#pragma unroll
+        for (int b = 0; b < 4; b++) sum += s_part[row / 4 * kS + i][m * kNN + n][at + 4 * b];
+      v[m] = (float)sum;
+    }
+    const int orow = first(blockIdx.x * kQ + row / 4) + row % 4;
+    f16_epilogue<kEpi, kNM>(v, r < rows_b, r, orow, row, w, o, qe, out16, w.mtiles, blockIdx.x);
   }
 }
 
@@ -2921,16 +3065,67 @@ bool launch_gemm_qkv(hipStream_t s, const MatrixView &w, const uint16_t *x, int 
   return true;
 }
 
-bool launch_matvec_swiglu_f16(hipStream_t s, const MatrixView &w, const ActView &act, int rows_b,
-                              const MatvecOut &o, uint16_t *out_f16) {
-  if (!g_prefill_mfma || rows_b < kPrefillRows || w.dtype != kFmtF16) return false;
-  return gemm_f16(s, kEpiSwiglu, w, act.f16, rows_b, o, out_f16);
+// The exact F16 kernels.  Up to 16 rows take k_mv_f16v: at 4 rows down (K
+// 4864) 5.9 us on eight waves per quad, 7.9 on four and 12 on two, sixteen no
+// better; gate+up (1,216 quads) 7.5 on four, 8.9 on eight.  Past 16 rows its
+// smaller tiles lose to k_mv_f16m (56 rows: down 27.4 against 16.4 us, gate+up
+// 36 against 25).  There, two batch tiles per workgroup share each weight
+// load and conversion where the grid still covers the CUs three times (92
+// rows: gate+up 39.3 against 41.5 us; head at 56 rows 324 against 359), one
+// otherwise (56 rows: down 16.1 against 25.9, gate+up 24.7 against 27.8);
+// four waves split K on large grids (56 rows: gate+up 24.7 against 27.4 on
+// eight), eight on small ones (down 16.1 against 18.3).
+template <int kEpi>
+static void mv_f16m(hipStream_t s, const MatrixView &w, const ActView &act, int rows_b, const MatvecOut &o,
+                    const QkvEpi &qe, uint16_t *out16) {
+  constexpr int kNM = kEpi == kEpiSwiglu || kEpi == kEpiQkv ? 2 : 1;
+  const int n_tiles = (rows_b + 15) / 16;
+  const int units = kEpi == kEpiSwiglu ? (w.rows / 2 + 15) / 16 : kEpi == kEpiQkv ? w.rows / 32 : w.mtiles;
+  auto go = [&](auto nn, auto kw) {
+    constexpr int kNN = decltype(nn)::value, kW = decltype(kw)::value;
+    const int ngroups = (n_tiles + kNN - 1) / kNN;
+    launch_k((k_mv_f16m<kEpi, kNM, kNN, kW>), dim3((units + 7) / 8 * 8 * ngroups), dim3(64 * kW),
+             (uint32_t)(kW * kNM * kNN * 16 * 17 * sizeof(double)), s, w, act, rows_b, n_tiles, o, qe, out16);
+  };
+  using std::integral_constant;
+  if (n_tiles == 1) {
+    const int quads = kEpi == kEpiSwiglu ? (w.rows / 2 + 3) / 4 : kEpi == kEpiQkv ? w.rows / 8 : (w.rows + 3) / 4;
+    auto small = [&](auto nn) {
+      constexpr int kNN = decltype(nn)::value;
+      auto run = [&](auto q, auto sp) {
+        constexpr int kQ = decltype(q)::value, kS = decltype(sp)::value;
+        launch_k((k_mv_f16v<kEpi, kNM, kNN, kQ, kS>), dim3((quads + kQ - 1) / kQ), dim3(64 * kQ * kS), 0, s, w, act,
+                 rows_b, o, qe, out16);
+      };
+      if constexpr (kEpi == kEpiArgmax)
+        run(integral_constant<int, 4>{}, integral_constant<int, 1>{});
+      else if (quads >= 1024)
+        run(integral_constant<int, 1>{}, integral_constant<int, 4>{});
+      else
+        run(integral_constant<int, 1>{}, integral_constant<int, 8>{});
+    };
+    switch ((rows_b + 3) / 4) {
+      case 1: return small(integral_constant<int, 1>{});
+      case 2: return small(integral_constant<int, 2>{});
+      case 3: return small(integral_constant<int, 3>{});
+      default: return small(integral_constant<int, 4>{});
+    }
+  }
+  const bool two = units * ((n_tiles + 1) / 2) >= 768;
+  const int groups = units * (two ? (n_tiles + 1) / 2 : n_tiles);
+  if (two && groups >= 1024)
+    go(integral_constant<int, 2>{}, integral_constant<int, 4>{});
+  else if (two)
+    go(integral_constant<int, 2>{}, integral_constant<int, 8>{});
+  else if (groups >= 1024)
+    go(integral_constant<int, 1>{}, integral_constant<int, 4>{});
+  else
+    go(integral_constant<int, 1>{}, integral_constant<int, 8>{});
 }
 
 template <int kEpi>
 static void mv_f16(hipStream_t s, const MatrixView &w, const ActView &act, int rows_b,
                    const MatvecOut &o) {
-  const int out_rows = kEpi == kEpiSwiglu ? w.rows / 2 : w.rows;
   // the head of a step in the packed-prefill regime (16+ logit rows): the
   // regime's GEMM with partial keys per 16-row tile
   if (kEpi == kEpiArgmax && g_head_mfma && rows_b >= 16 &&
@@ -2941,16 +3136,19 @@ static void mv_f16(hipStream_t s, const MatrixView &w, const ActView &act, int r
   if ((kEpi == kEpiStore || kEpi == kEpiResidual) && g_prefill_mfma && rows_b >= kPrefillRows &&
       gemm_f16(s, (Epilogue)kEpi, w, act.f16, rows_b, o, nullptr))
     return;
-  if (rows_b >= 16 && w.K % 8 == 0) {  // lane = batch row, sequential f64 chains
-    launch_k(k_mv_f16s<kEpi>, dim3((out_rows + 15) / 16, (rows_b + kWave - 1) / kWave), dim3(256), 0,
-             s, w, act, rows_b, o);
-    return;
-  }
-  if (kEpi == kEpiArgmax) {  // partial keys per 16-row tile, then k_argmax_reduce
-    launch_k(k_head_f16, dim3(w.mtiles), dim3(256), 0, s, w, act, rows_b, o);
-    return;
-  }
-  launch_k(k_mv_f16<kEpi>, dim3((out_rows + 3) / 4), dim3(256), 0, s, w, act, rows_b, o);
+  if (w.K % 32 == 0)
+    mv_f16m<kEpi>(s, w, act, rows_b, o, QkvEpi{}, nullptr);
+  else if constexpr (kEpi == kEpiStore)  // cohx_matvec alone takes such widths
+    launch_k(k_mv_f16, dim3((w.rows + 3) / 4), dim3(256), 0, s, w, act, rows_b, o);
+}
+
+bool launch_matvec_swiglu_f16(hipStream_t s, const MatrixView &w, const ActView &act, int rows_b,
+                              const MatvecOut &o, uint16_t *out_f16) {
+  if (w.dtype != kFmtF16) return false;
+  if (g_prefill_mfma && rows_b >= kPrefillRows && gemm_f16(s, kEpiSwiglu, w, act.f16, rows_b, o, out_f16)) return true;
+  if (w.K % 32) return false;
+  mv_f16m<kEpiSwiglu>(s, w, act, rows_b, o, QkvEpi{}, out_f16);
+  return true;
 }
 
 template <int kEpi, int kNM>
@@ -2997,6 +3195,7 @@ bool launch_matvec(hipStream_t s, Epilogue epi, const MatrixView &w, const ActVi
 void launch_matvec_qkv(hipStream_t s, const MatrixView &w, const ActView &act, int rows_b,
                        const MatvecOut &o, const QkvEpi &q) {
   const int n_tiles = (rows_b + 15) / 16, groups = (w.mtiles + 7) / 8;
+  if (w.dtype == kFmtF16) return mv_f16m<kEpiQkv>(s, w, act, rows_b, o, q, nullptr);
   if (n_tiles <= 2 && w.dtype == 8)  // as for the residual projections, below 3 batch tiles
     launch_k((k_mv_q8s<kEpiQkv, 1, 2, 8, 16>), dim3(groups * 8 * n_tiles), dim3(1024), 0, s, w, act, rows_b,
              n_tiles, o, q);
