@@ -614,12 +614,41 @@ __global__ __launch_bounds__(256) void k_q35_gates(const float *__restrict__ con
   }
 }
 
-// The recurrence: one workgroup per (lane, value head); thread j keeps state
-// column j (kKD cells) in registers across the lane's tokens.  Per token the
-// cells decay, the prediction chain sum_i f64(cell * k_i*k_scale) runs in key
-// order from +0.0, corr = (v_j - f32(pred)) * beta, then the cells take
-// k_i*k_scale*corr and the read chain sum_i f64(cell * q_i*q_scale) gives
-// the head's raw output.
+// Sum of v over aligned groups of kP lanes (1, 2, 4 or 8), the same bits in
+// each lane: neighbours, then pairs, then fours.
+template <int kCtrl>
+__device__ __forceinline__ double dpp_f64(double v) {
+  const uint64_t u = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, kCtrl, 0xf, 0xf, false);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), kCtrl, 0xf, 0xf, false);
+  return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+}
+template <int kP>
+__device__ __forceinline__ double parts_sum(double v) {
+  if constexpr (kP >= 2) v += dpp_f64<0xB1>(v);   // quad_perm [1,0,3,2]
+  if constexpr (kP >= 4) v += dpp_f64<0x4E>(v);   // quad_perm [2,3,0,1]
+  if constexpr (kP >= 8) v += dpp_f64<0x141>(v);  // row_half_mirror
+  return v;
+}
+
+// The recurrence over prompt chunks.  kP lanes own one state column, 16 keys
+// each (in registers across the lane's tokens); a workgroup of 256 threads
+// owns 256 / kP columns of one (lane, value head).  Per token the cells decay,
+// the prediction sum_i f64(cell * k_i*k_scale) runs in key order from +0.0
+// within each lane's 16 keys and over the lanes in a fixed tree, corr =
+// (v_j - f32(pred)) * beta, then the cells take k_i*k_scale*corr and the read
+// sum_i f64(cell * q_i*q_scale) gives the head's raw output.  (The reference
+// runs each f64 sum as one chain, kernels.rs:122-214.  Its terms are f32
+// products of 24 bits, so a partial sum rounds only where a term is 2^-29 of
+// it or smaller, by 2^-53 of its size, before the sum is rounded to f32.)
+//   What bounds it: vector issue, five f32 and four f64 operations a cell and
+// token (about 0.9 us a token and CU at full rate).  One thread per column,
+// two waves a CU, took 3.0 us a token; sixteen waves a CU cover the
+// operations' latencies.  The key vectors, values and gates of kT tokens are
+// staged in LDS at a time, the next kT requested while they are used, so there
+// is one barrier per kT tokens.  Workgroups of one column group start at
+// another lane (blockIdx.z), so a CU's share mixes long and short lanes.
+// Measured at 16 lanes of 64-449 tokens: 1,345 -> 444 us a launch.
 template <int kKD>
 __global__ __launch_bounds__(256) void k_q35_delta(Q35Lanes L, const float *__restrict__ conv,
                                                    int ldc, int keys,
@@ -627,120 +656,108 @@ __global__ __launch_bounds__(256) void k_q35_delta(Q35Lanes L, const float *__re
                                                    int VH, int VD, float *state, size_t state_seq,
                                                    float *__restrict__ o_out, int ldo,
                                                    uint32_t *row_err) {
-  __shared__ __align__(16) float s_qq[kKD], s_kk[kKD];
-  const int ln = blockIdx.x, h = blockIdx.y, j = threadIdx.x;
+  constexpr int kP = kKD / 16, kC = 256 / kP;  // lanes per column, columns per workgroup
+  constexpr int kT = 8;                        // tokens per stage
+  constexpr int kSK = 2 * kKD * kT / 256, kSV = kC * kT / 256;  // staged key and value words per thread
+  // keys as [quad][lane of the column][4]: the kP lanes of a column read
+  // consecutive 16-byte words
+  __shared__ __align__(16) float s_k[2][kT][kKD], s_q[2][kT][kKD], s_v[2][kT][kC];
+  __shared__ float4 s_g[2][kT];
+  const int tid = threadIdx.x, h = blockIdx.y;
+  const int nl = gridDim.x, ln = (int)(blockIdx.x + blockIdx.z * (nl / gridDim.z)) % nl;
   const uint32_t first = L.first[ln], n = L.n[ln];
-  const int src = (h / (VH / KH)) * kKD;
-  float *S = state + (size_t)L.seq[ln] * state_seq + (size_t)h * kKD * VD;
+  if (!n) return;
+  const int src = (h / (VH / KH)) * kKD, j0 = blockIdx.z * kC;
+  const int part = tid % kP, c = tid / kP, j = j0 + c;
   const bool active = j < VD;
-  // the column moves through a buffer resource: lane offset j*4 in one VGPR,
-  // key offset i*VD*4 as a scalar, so no per-key address stays live
-  const __amdgpu_buffer_rsrc_t rs =
-      __builtin_amdgcn_make_buffer_rsrc(S, (short)0, (int)(kKD * VD * 4), 0x00020000);
-  const int voff = active ? j * 4 : 0;
-  float col[kKD];
+  float *S = state + (size_t)L.seq[ln] * state_seq + (size_t)h * kKD * VD + (active ? j : 0);
+  float col[16];
 #pragma unroll
-  for (int i = 0; i < kKD; i++)
-    col[i] = active ? __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, voff, i * VD * 4, 0))
-                    : 0.0f;
-  // token t + 1's gates, q/k channel j and v channel j are requested while
-  // token t's chains run (the launcher gives at least kKD threads)
-  float4 gt_n = make_float4(0.f, 0.f, 0.f, 0.f);
-  float q_n = 0.0f, k_n = 0.0f, v_n = 0.0f;
-  auto fetch = [&](uint32_t t) {
-    const float *cr = conv + (size_t)(first + t) * ldc;
-    gt_n = gates[(size_t)(first + t) * VH + h];
-    if (j < kKD) {
-      q_n = cr[src + j];
-      k_n = cr[keys + src + j];
+  for (int i = 0; i < 16; i++) col[i] = active ? S[(size_t)(16 * part + i) * VD] : 0.0f;
+  // word e = tid + 256 i of a stage's keys: token e / (2 kKD), then q and k channels
+  float rk[kSK], rs[kSK], rv[kSV];
+  float4 rg = make_float4(0.f, 0.f, 0.f, 0.f);
+  auto fetch = [&](uint32_t t0) {
+#pragma unroll
+    for (int i = 0; i < kSK; i++) {
+      const int e = tid + 256 * i, t = e / (2 * kKD), ch = e % (2 * kKD);
+      const size_t row = first + min(t0 + t, n - 1);
+      rk[i] = conv[row * ldc + (ch < kKD ? src + ch : keys + src + ch - kKD)];
+      const float4 &g = gates[row * VH + h];
+      rs[i] = ch < kKD ? g.x : g.y;
     }
-    if (active) v_n = cr[2 * keys + h * VD + j];
+#pragma unroll
+    for (int i = 0; i < kSV; i++) {
+      const int e = tid + 256 * i, t = e / kC, cc = e % kC;
+      const size_t row = first + min(t0 + t, n - 1);
+      rv[i] = j0 + cc < VD ? conv[row * ldc + 2 * keys + h * VD + j0 + cc] : 0.0f;
+    }
+    if (tid < kT) rg = gates[(size_t)(first + min(t0 + tid, n - 1)) * VH + h];
   };
-  if (n) fetch(0);
-  for (uint32_t t = 0; t < n; t++) {
-    const uint32_t row = first + t;
-    const float4 gt = gt_n;
-    const float qc = q_n, kc = k_n, v = v_n;
+  auto stash = [&](int buf) {
+#pragma unroll
+    for (int i = 0; i < kSK; i++) {
+      const int e = tid + 256 * i, t = e / (2 * kKD), ch = e % (2 * kKD), k = ch % kKD;
+      const int at = ((k % 16 / 4) * kP + k / 16) * 4 + k % 4;
+      (ch < kKD ? s_q : s_k)[buf][t][at] = rk[i] * rs[i];
+    }
+#pragma unroll
+    for (int i = 0; i < kSV; i++) {
+      const int e = tid + 256 * i;
+      s_v[buf][e / kC][e % kC] = rv[i];
+    }
+    if (tid < kT) s_g[buf][tid] = rg;
+  };
+  fetch(0);
+  stash(0);
+  __syncthreads();
+  int buf = 0;
+  for (uint32_t t0 = 0; t0 < n; t0 += kT) {
+    const bool more = t0 + kT < n;
+    if (more) fetch(t0 + kT);
+    const int nt = (int)min((uint32_t)kT, n - t0);
+    for (int t = 0; t < nt; t++) {
+      const float4 gt = s_g[buf][t];
+      const float v = s_v[buf][t][c], decay = gt.z, beta = gt.w;
+      float kk[16], qq[16];
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        const float4 a = *reinterpret_cast<const float4 *>(&s_k[buf][t][(u * kP + part) * 4]);
+        const float4 b = *reinterpret_cast<const float4 *>(&s_q[buf][t][(u * kP + part) * 4]);
+        kk[4 * u] = a.x; kk[4 * u + 1] = a.y; kk[4 * u + 2] = a.z; kk[4 * u + 3] = a.w;
+        qq[4 * u] = b.x; qq[4 * u + 1] = b.y; qq[4 * u + 2] = b.z; qq[4 * u + 3] = b.w;
+      }
+      double pred = 0.0;
+#pragma unroll
+      for (int i = 0; i < 16; i++) {
+        col[i] *= decay;
+        pred += (double)(col[i] * kk[i]);
+      }
+      pred = parts_sum<kP>(pred);
+      const float corr = (v - (float)pred) * beta;
+      double rd = 0.0;
+#pragma unroll
+      for (int i = 0; i < 16; i++) {
+        col[i] += kk[i] * corr;
+        rd += (double)(col[i] * qq[i]);
+      }
+      const float o = (float)parts_sum<kP>(rd);
+      // a non-finite cell makes its read product non-finite (inf * 0 is NaN),
+      // and no f64 sum brings an inf or NaN term back to a finite value, so o
+      // is non-finite whenever any updated cell is: o covers the cells' check
+      if (active && part == 0) {
+        const size_t row = first + t0 + t;
+        o_out[row * ldo + h * VD + j] = o;
+        if (!finitef(o) || !finitef(v)) atomicOr(&row_err[row], kErrRequest);
+      }
+    }
+    if (more) stash(buf ^ 1);
     __syncthreads();
-    if (j < kKD) {
-      s_qq[j] = qc * gt.x;
-      s_kk[j] = kc * gt.y;
-    }
-    if (t + 1 < n) fetch(t + 1);
-    __syncthreads();
-    if (!active) continue;
-    const float decay = gt.z, beta = gt.w;
-    // the keys' LDS values are requested two groups of 4 ahead of their use,
-    // so the chains do not wait on LDS at every group
-    const float4 *kk4 = reinterpret_cast<const float4 *>(s_kk);
-    const float4 *qq4 = reinterpret_cast<const float4 *>(s_qq);
-    constexpr int kG4 = kKD / 4;
-    double pred = 0.0;
-    float4 ka = kk4[0], kb = kG4 > 1 ? kk4[1] : ka;
-#pragma unroll
-    for (int i0 = 0; i0 < kKD; i0 += 4) {
-      asm volatile("" ::: "memory");
-      const float4 kq = ka;
-      ka = kb;
-      if (i0 / 4 + 2 < kG4) kb = kk4[i0 / 4 + 2];
-      const float kv[4] = {kq.x, kq.y, kq.z, kq.w};
-      float p[4];
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        col[i0 + e] *= decay;
-        p[e] = col[i0 + e] * kv[e];
-      }
-      pin_vgprs(p);
-      double wd[4];
-#pragma unroll
-      for (int e = 0; e < 4; e++) wd[e] = (double)p[e];
-      pin_vgprs(wd);
-#pragma unroll
-      for (int e = 0; e < 4; e++) pred += wd[e];
-    }
-    const float corr = (v - (float)pred) * beta;
-    double rd = 0.0;
-    ka = kk4[0];
-    kb = kG4 > 1 ? kk4[1] : ka;
-    float4 qa = qq4[0], qb = kG4 > 1 ? qq4[1] : qa;
-#pragma unroll
-    for (int i0 = 0; i0 < kKD; i0 += 4) {
-      asm volatile("" ::: "memory");
-      const float4 kq = ka, qv4 = qa;
-      ka = kb;
-      qa = qb;
-      if (i0 / 4 + 2 < kG4) {
-        kb = kk4[i0 / 4 + 2];
-        qb = qq4[i0 / 4 + 2];
-      }
-      const float kv[4] = {kq.x, kq.y, kq.z, kq.w}, qv[4] = {qv4.x, qv4.y, qv4.z, qv4.w};
-      float p[4];
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        col[i0 + e] += kv[e] * corr;
-        p[e] = col[i0 + e] * qv[e];
-      }
-      pin_vgprs(p);
-      double wd[4];
-#pragma unroll
-      for (int e = 0; e < 4; e++) wd[e] = (double)p[e];
-      pin_vgprs(wd);
-#pragma unroll
-      for (int e = 0; e < 4; e++) rd += wd[e];
-    }
-    const float o = (float)rd;
-    // a non-finite cell makes its read product non-finite (inf * 0 is NaN),
-    // and no f64 sum brings an inf or NaN term back to a finite value, so o
-    // is non-finite whenever any updated cell is: o covers the cells' check
-    const bool bad = !finitef(o) || !finitef(v);
-    o_out[(size_t)row * ldo + h * VD + j] = o;
-    if (bad) atomicOr(&row_err[row], kErrRequest);
+    buf ^= 1;
   }
   if (active) {
 #pragma unroll
-    for (int i = 0; i < kKD; i++)
-      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, col[i]), rs, voff,
-                                            i * VD * 4, 0);
+    for (int i = 0; i < 16; i++) S[(size_t)(16 * part + i) * VD] = col[i];
   }
 }
 
@@ -1390,13 +1407,12 @@ void q35_delta(hipStream_t s, int rows, int lanes, Q35Lanes L, const float *conv
                float *o_raw, float *tgt, int ldt, uint32_t *row_err) {
   hipLaunchKernelGGL(k_q35_gates, dim3(rows, value_heads), dim3(128), 0, s, conv, ldc, keys, mix,
                      ldm, a_off, b_off, a_log, dt, key_heads, value_heads, key_dim, gates, row_err);
-  // at least key_dim threads: thread j stages q/k channel j of each token
-  const dim3 grid(lanes, value_heads),
-      block(((std::max(value_dim, key_dim) + kWave - 1) / kWave) * kWave);
+  const dim3 block(((value_dim + kWave - 1) / kWave) * kWave);
 #define L_(KD)                                                                                 \
   case KD:                                                                                     \
-    hipLaunchKernelGGL(k_q35_delta<KD>, grid, block, 0, s, L, conv, ldc, keys, gates, key_heads, \
-                       value_heads, value_dim, state, state_seq, o_raw, ldt, row_err);         \
+    hipLaunchKernelGGL(k_q35_delta<KD>, dim3(lanes, value_heads, (value_dim + 4096 / KD - 1) / (4096 / KD)), \
+                       dim3(256), 0, s, L, conv, ldc, keys, gates, key_heads, value_heads, value_dim, state, \
+                       state_seq, o_raw, ldt, row_err);                                        \
     break;
   switch (key_dim) {
     L_(16) L_(32) L_(64) L_(128)
