@@ -608,7 +608,7 @@ int q35_step(cohx_ctx *ctx, const cohx_batch *batch, cohx_step_out *out, const c
                    q->delta_state + (size_t)Ly.slot * q->VH * q->KD * q->VD, q->delta_seq, q->tgt,
                    q->ld_att, q->row_err);
       } else {
-        q35_conv(s, NL, L, q->mix_out, q->ld_mix, Ly.conv, q->C, q->K,
+        q35_conv(s, NL, (int)max_lane_tokens, L, q->mix_out, q->ld_mix, Ly.conv, q->C, q->K,
                  q->conv_state + (size_t)Ly.slot * q->C * q->K, q->conv_seq, q->cv, q->C,
                  q->row_err);
         q35_delta(s, (int)R, NL, L, q->cv, q->C, q->keys, q->mix_out, q->ld_mix, q->lin_z,

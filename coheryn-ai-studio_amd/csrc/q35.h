@@ -73,7 +73,8 @@ bool q35_matvec_swiglu(hipStream_t s, const uint16_t *w, int up_off, int F, int 
                        int ldx, int R, float *h, int ldh, uint32_t *row_err);
 void q35_swiglu(hipStream_t s, int rows, const float *gu, int ldgu, int F, int up_off, float *h,
                 int ldh);
-void q35_conv(hipStream_t s, int lanes, Q35Lanes L, const float *mix, int ldm, const float *w,
+// max_tokens: the most tokens any lane carries.
+void q35_conv(hipStream_t s, int lanes, int max_tokens, Q35Lanes L, const float *mix, int ldm, const float *w,
               int C, int K, float *hist, size_t hist_seq, float *out, int ldo, uint32_t *row_err);
 bool q35_delta_supported(int key_dim, int value_dim);
 // The whole linear-attention mixer (conv, gates, delta rule, output norm x

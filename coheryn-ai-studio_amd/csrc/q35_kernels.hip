@@ -30,6 +30,11 @@ __device__ __forceinline__ float sigmoid_f32(float x) {
   return e / (1.0f + e);
 }
 __device__ __forceinline__ float silu_f32(float x) { return x * sigmoid_f32(x); }
+// The same with expf's table staged in LDS (per-lane reads).
+__device__ __forceinline__ float silu_f32(float x, const uint64_t *tab) {
+  const float e = exp_f32_tab(-fabsf(x), tab);
+  return x * (x >= 0.0f ? 1.0f / (1.0f + e) : e / (1.0f + e));
+}
 __device__ __forceinline__ float softplus_f32(float x) {
   return fmaxf(x, 0.0f) + log1p_f32(exp_f32(-fabsf(x)));
 }
@@ -506,69 +511,89 @@ __global__ __launch_bounds__(256) void k_q35_swiglu(const float *__restrict__ gu
 }
 
 // ---------------------------------------------------------------------------
-// Causal depthwise conv (kernels.rs:54-120), one thread per channel walking
-// its lane's tokens in order.  The ring is kept in time order in registers
-// (oldest first), which is exactly the reference's slot order
-// (cursor + 1 + i) % kernel after the new input is written; the cursor of a
-// sequence is position % kernel, since every layer steps once per token.
+// Causal depthwise conv (kernels.rs:54-120).  An output needs its channel's
+// last K inputs only, so a lane's tokens are cut into segments of kConvSeg: a
+// workgroup takes 256 channels of one segment, its first taps coming from the
+// rows before the segment (from the ring for a lane's first tokens).  The ring
+// is in time order, oldest first, from slot position % kernel on, which is the
+// reference's slot order (cursor + 1 + i) % kernel after the new input is
+// written (every layer steps once per token).  The lane's first segment alone
+// reads the ring and, when its tokens are done, leaves the lane's last inputs
+// in it.
+//   What bounds it: one read and one write of the rows.  One thread per
+// channel walking its lane's tokens waited on memory once per eight tokens:
+// 332 us a launch at 16 lanes of 64-449 tokens, 64 now (143 with run-time
+// widths and expf's table in constant memory).
 // ---------------------------------------------------------------------------
-constexpr int kMaxConv = 8;
+constexpr int kMaxConv = 8, kConvSeg = 32;
+template <int kK>  // the kernel width, or 0: any up to kMaxConv
 __global__ __launch_bounds__(256) void k_q35_conv(Q35Lanes L, const float *__restrict__ mix,
                                                   int ldm, const float *__restrict__ w, int C,
-                                                  int K, float *hist, size_t hist_seq,
+                                                  int K_, float *hist, size_t hist_seq,
                                                   float *__restrict__ out, int ldo,
                                                   uint32_t *row_err) {
+  constexpr int kTaps = kK ? kK : kMaxConv;
+  const int K = kK ? kK : K_;
+  __shared__ uint64_t s_tab[32];
+  if (threadIdx.x < 32) s_tab[threadIdx.x] = kExp2Tab[threadIdx.x];
+  __syncthreads();
   const int ln = blockIdx.x, ch = blockIdx.y * 256 + threadIdx.x;
-  if (ch >= C) return;
   const uint32_t first = L.first[ln], n = L.n[ln], start = L.start[ln];
+  const uint32_t seg = blockIdx.z * kConvSeg, end = min(n, seg + kConvSeg);
+  if (ch >= C || seg >= n) return;
   float *h = hist + (size_t)L.seq[ln] * hist_seq + (size_t)ch * K;
   const int c0 = (int)(start % (uint32_t)K);
-  float tap[kMaxConv], wv[kMaxConv];
+  const float *mc = mix + ch;
+  // the K inputs before token seg, oldest first: ring entries (of which the
+  // oldest is dropped by the first token) or earlier rows
+  static_assert(kConvSeg >= kMaxConv, "a later segment's taps are rows of the lane");
+  float tap[kTaps], wv[kTaps];
 #pragma unroll
-  for (int i = 0; i < kMaxConv; i++) {
-    tap[i] = i < K ? h[(c0 + i) % K] : 0.0f;
+  for (int i = 0; i < kTaps; i++) {
+    tap[i] = i >= K ? 0.0f : seg == 0 ? h[(c0 + i) % K] : mc[(size_t)(first + seg - K + i) * ldm];
     wv[i] = i < K ? w[(size_t)ch * K + i] : 0.0f;
   }
   // the inputs load a group of kAhead tokens at a time, the next group
-  // requested before the current one is folded in, so a chunk's walk waits
-  // on memory once per group rather than once per token
+  // requested before the current one is folded in
   constexpr int kAhead = 8;
-  const float *mc = mix + ch;
   float cur[kAhead], nxt[kAhead];
 #pragma unroll
-  for (int j = 0; j < kAhead; j++) cur[j] = (uint32_t)j < n ? mc[(size_t)(first + j) * ldm] : 0.0f;
-  for (uint32_t t0 = 0; t0 < n; t0 += kAhead) {
+  for (int j = 0; j < kAhead; j++) cur[j] = seg + j < end ? mc[(size_t)(first + seg + j) * ldm] : 0.0f;
+  for (uint32_t t0 = seg; t0 < end; t0 += kAhead) {
 #pragma unroll
     for (int j = 0; j < kAhead; j++) {
       const uint32_t tn = t0 + kAhead + j;
-      nxt[j] = tn < n ? mc[(size_t)(first + tn) * ldm] : 0.0f;
+      nxt[j] = tn < end ? mc[(size_t)(first + tn) * ldm] : 0.0f;
     }
 #pragma unroll
     for (int j = 0; j < kAhead; j++) {
-      if (t0 + j >= n) break;
+      if (t0 + j >= end) break;
       const uint32_t row = first + t0 + j;
       const float in = cur[j];
 #pragma unroll
-      for (int i = 0; i < kMaxConv - 1; i++)
+      for (int i = 0; i < kTaps - 1; i++)
         if (i < K - 1) tap[i] = tap[i + 1];
 #pragma unroll
-      for (int i = 0; i < kMaxConv; i++)
+      for (int i = 0; i < kTaps; i++)
         if (i == K - 1) tap[i] = in;
       double sum = -0.0;
 #pragma unroll
-      for (int i = 0; i < kMaxConv; i++)
+      for (int i = 0; i < kTaps; i++)
         if (i < K) sum += (double)(tap[i] * wv[i]);
-      const float y = silu_f32((float)sum);
+      const float y = silu_f32((float)sum, s_tab);
       out[(size_t)row * ldo + ch] = y;
       if (!finitef(in) || !finitef(y)) atomicOr(&row_err[row], kErrRequest);
     }
 #pragma unroll
     for (int j = 0; j < kAhead; j++) cur[j] = nxt[j];
   }
+  if (seg != 0) return;
+  // the lane's last K inputs: rows, or what is left of the ring before them
+  // (n < K, where the lane is this one segment and tap holds them)
   const int c1 = (int)((start + n) % (uint32_t)K);
 #pragma unroll
-  for (int i = 0; i < kMaxConv; i++)
-    if (i < K) h[(c1 + i) % K] = tap[i];
+  for (int i = 0; i < kTaps; i++)
+    if (i < K) h[(c1 + i) % K] = n >= (uint32_t)K ? mc[(size_t)(first + n - K + i) * ldm] : tap[i];
 }
 
 // ---------------------------------------------------------------------------
@@ -1365,10 +1390,13 @@ void q35_swiglu(hipStream_t s, int rows, const float *gu, int ldgu, int F, int u
                      up_off, h, ldh);
 }
 
-void q35_conv(hipStream_t s, int lanes, Q35Lanes L, const float *mix, int ldm, const float *w,
+void q35_conv(hipStream_t s, int lanes, int max_tokens, Q35Lanes L, const float *mix, int ldm, const float *w,
               int C, int K, float *hist, size_t hist_seq, float *out, int ldo, uint32_t *row_err) {
-  hipLaunchKernelGGL(k_q35_conv, dim3(lanes, (C + 255) / 256), dim3(256), 0, s, L, mix, ldm, w, C,
-                     K, hist, hist_seq, out, ldo, row_err);
+  const dim3 grid(lanes, (C + 255) / 256, (max_tokens + kConvSeg - 1) / kConvSeg);
+  if (K == 4)
+    hipLaunchKernelGGL(k_q35_conv<4>, grid, dim3(256), 0, s, L, mix, ldm, w, C, K, hist, hist_seq, out, ldo, row_err);
+  else
+    hipLaunchKernelGGL(k_q35_conv<0>, grid, dim3(256), 0, s, L, mix, ldm, w, C, K, hist, hist_seq, out, ldo, row_err);
 }
 
 bool q35_linear_fused(int conv_kernel, int key_heads, int value_heads) {
