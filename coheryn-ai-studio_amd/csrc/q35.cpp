@@ -632,8 +632,9 @@ int q35_step(cohx_ctx *ctx, const cohx_batch *batch, cohx_step_out *out, const c
         return lrc;
     }
     q35_norm(s, (int)R, q->x, H, nullptr, Ly.post_norm, H, eps, 1, q->nrm, H, q->row_err, nullptr);
-    if (regime || !q35_matvec_swiglu(s, Ly.gu, q->gu_up, q->F, H, q->nrm, H, (int)R, q->hb, q->F,
-                                     q->row_err)) {
+    if (!regime) {
+      q35_matvec_swiglu(s, Ly.gu, q->gu_up, q->F, H, q->nrm, H, (int)R, q->hb, q->row_err);
+    } else {
       if ((lrc = linear(kQ35Store, Ly.gu, q->gu_rows, q->gu_rows, H, q->nrm, H, q->gu_out,
                         q->gu_rows)))
         return lrc;

@@ -47,8 +47,8 @@ void q35_embed(hipStream_t s, int rows, const uint16_t *embed, const uint32_t *t
 void q35_norm(hipStream_t s, int rows, const float *x, int ldx, const uint32_t *src,
               const float *w, int n, float eps, int zc, float *out, int ldo, uint32_t *row_err,
               const uint32_t *err_row);
-// out[r][o] (=, +=) sum_k x[r][k] * w[o][k] in f64, k in order; argmax keys
-// per 64-output block go to part[r][block] (logits optional).
+// out[r][o] (=, +=) sum_k f32(x[r][k] * w[o][k]) in f64, in a fixed order;
+// argmax keys per 16-output tile go to part[r][tile] (logits optional).
 void q35_matvec(hipStream_t s, int epi, const uint16_t *w, int rows_w, int valid_rows, int K,
                 const float *x, int ldx, int R, float *out, int ldo, unsigned long long *part,
                 uint32_t *row_err, const uint32_t *err_row);
@@ -64,13 +64,11 @@ void q35_split_bf16(hipStream_t s, int rows, int K, const float *x, int ldx, uin
 // non-finite output.
 void q35_gemm_split(hipStream_t s, bool accumulate, const uint16_t *w, int N, int K, const uint16_t *hi,
                     const uint16_t *lo, int rows, float *out, int ldo, uint32_t *row_err);
-// Gate+up and SwiGLU in one launch for few rows: h[r][f] = silu(gate) * up
-// with the bits of q35_matvec (gate rows [0, F), up rows [up_off, up_off + F))
-// followed by q35_swiglu.  Returns false (nothing launched) where q35_matvec
-// would not take its one-chain-per-lane form (more than 64 rows, or few
-// enough tiles for the producer/consumer form).
-bool q35_matvec_swiglu(hipStream_t s, const uint16_t *w, int up_off, int F, int K, const float *x,
-                       int ldx, int R, float *h, int ldh, uint32_t *row_err);
+// Gate+up and SwiGLU in one launch: h[r][f] = silu(gate) * up with the bits of
+// q35_matvec (gate rows [0, F), up rows [up_off, up_off + F), up_off a multiple
+// of 16) followed by q35_swiglu.
+void q35_matvec_swiglu(hipStream_t s, const uint16_t *w, int up_off, int F, int K, const float *x,
+                       int ldx, int R, float *h, uint32_t *row_err);
 void q35_swiglu(hipStream_t s, int rows, const float *gu, int ldgu, int F, int up_off, float *h,
                 int ldh);
 // max_tokens: the most tokens any lane carries.

@@ -11,6 +11,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "device.h"
 #include "gemm.h"
@@ -19,6 +20,8 @@
 
 namespace cohx {
 namespace {
+
+typedef unsigned int u32x4q __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ float bf_lo(uint32_t w) { return __uint_as_float(w << 16); }
 __device__ __forceinline__ float bf_hi(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
@@ -136,361 +139,170 @@ __global__ __launch_bounds__(256) void k_q35_norm(const float *__restrict__ x, i
 
 // ---------------------------------------------------------------------------
 // BF16 matvec (tensor.rs:380-406 -> cpu::dot): out[r][o] = f32(sum_k
-// f64(w[o][k] * x[r][k])), k in order from -0.0.  A workgroup owns 64
-// outputs (4 tiles of 16, one per wave) x 16 batch rows staged in LDS; lane
-// (o16, g) runs rows 4g..4g+3 of output o16 as four chains, issued as pinned
-// groups of products, widenings and adds.
+// f64(f32(w[o][k] * x[r][k]))).  A workgroup owns one tile of 16 outputs x kR
+// rows; its kW waves take 64-input chunks in turn, and within a chunk each
+// 16-lane row of the wave takes 16 inputs: lane l brings the weights of
+// output l % 16 (two 16-byte loads, coalesced in the tile layout).  The rows'
+// inputs pass through a strip of LDS of the wave's own (256 contiguous bytes a
+// row, no barrier: a wave's LDS operations stay in order) and come back as
+// 16-byte broadcasts.  The 4 kW partial sums of an output meet in LDS and are
+// added in a fixed order.  (The reference adds the products in one chain.
+// They are f32 values of 24 bits, so a partial f64 sum rounds only where a
+// product is 2^-29 of it or smaller, by 2^-53 of its size, before the dot is
+// rounded to f32.)
+//   What bounds it: vector issue, an f32 multiply, a widening and an f64 add
+// per product, 4.6 ns a wave and SIMD, issued as pinned groups of products,
+// widenings and adds over up to eight rows (left alone, the compiler sends
+// every triple through one temporary and each add waits for its widening;
+// taking the inputs from the lanes by DPP, without LDS, cost 5.9 ns).  One chain per output left a decode
+// step waiting on 1,024 to 3,584 dependent adds in every linear.
+//   kQ35Swiglu: gate tile blockIdx.x and up tile blockIdx.x + up_off / 16
+// (up_off passed in valid_rows, F in ldo's place as the output count) over the
+// same inputs; h = (g / (1 + exp(-g))) * u (the SwiGLU pass's expression) to
+// out [R][F].
+//   Measured at 16 rows (us a launch, one chain per output before): o 7.3 and
+// down 10.0 (22.4 each), mix 17.1 (22.2), gate+up 15.0 (18.3), head 340 (343);
+// o and down at 96 rows 28 on average (228).
 // ---------------------------------------------------------------------------
-constexpr int kMvRows = 16, kMvKC = 256;
-template <int kEpi>
-__global__ __launch_bounds__(256) void k_q35_mv(const uint16_t *__restrict__ w, int rows_w,
-                                                int valid_rows, int K,
-                                                const float *__restrict__ x, int ldx, int R,
-                                                float *out, int ldo,
-                                                unsigned long long *__restrict__ part,
-                                                uint32_t *row_err,
-                                                const uint32_t *__restrict__ err_row) {
-  // rows padded by 4 floats: the four row groups of a wave read different banks
-  __shared__ __align__(16) float xs[kMvRows][kMvKC + 4];
-  __shared__ unsigned long long keys[kMvRows][64];
-  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-  const int o16 = lane % 16, g = lane / 16;
-  const int tile = blockIdx.x * 4 + wave, r0 = blockIdx.y * kMvRows;
-  const int o = tile * 16 + o16;
-  const bool live_tile = tile * 16 < rows_w;
-  const uint4 *wt = reinterpret_cast<const uint4 *>(w) + (size_t)tile * (K / 8) * 16 + o16;
-  double acc[4] = {-0.0, -0.0, -0.0, -0.0};
-  for (int k0 = 0; k0 < K; k0 += kMvKC) {
-    const int kc = min(kMvKC, K - k0);
-    __syncthreads();
-    for (int i = threadIdx.x; i < kMvRows * (kMvKC / 4); i += 256) {
-      const int rr = i / (kMvKC / 4), c4 = (i % (kMvKC / 4)) * 4;
-      float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-      if (r0 + rr < R && c4 < kc)
-        v = *reinterpret_cast<const float4 *>(x + (size_t)(r0 + rr) * ldx + k0 + c4);
-      *reinterpret_cast<float4 *>(&xs[rr][c4]) = v;
-    }
-    __syncthreads();
-    if (!live_tile) continue;
-    for (int kk = 0; kk < kc; kk += 8) {
-      const uint4 wv = wt[(size_t)((k0 + kk) / 8) * 16];
-      const float wf[8] = {bf_lo(wv.x), bf_hi(wv.x), bf_lo(wv.y), bf_hi(wv.y),
-                           bf_lo(wv.z), bf_hi(wv.z), bf_lo(wv.w), bf_hi(wv.w)};
-      float xv[4][8];
-#pragma unroll
-      for (int rr = 0; rr < 4; rr++) {
-        const float4 lo = *reinterpret_cast<const float4 *>(&xs[g * 4 + rr][kk]);
-        const float4 hi = *reinterpret_cast<const float4 *>(&xs[g * 4 + rr][kk + 4]);
-        xv[rr][0] = lo.x; xv[rr][1] = lo.y; xv[rr][2] = lo.z; xv[rr][3] = lo.w;
-        xv[rr][4] = hi.x; xv[rr][5] = hi.y; xv[rr][6] = hi.z; xv[rr][7] = hi.w;
-      }
-#pragma unroll
-      for (int e = 0; e < 8; e++) {
-        float pr[4];
-#pragma unroll
-        for (int rr = 0; rr < 4; rr++) pr[rr] = wf[e] * xv[rr][e];
-        pin_vgprs(pr);
-        double wd[4];
-#pragma unroll
-        for (int rr = 0; rr < 4; rr++) wd[rr] = (double)pr[rr];
-        pin_vgprs(wd);
-#pragma unroll
-        for (int rr = 0; rr < 4; rr++) acc[rr] += wd[rr];
-        pin_vgprs(acc);
-      }
-    }
-  }
-#pragma unroll
-  for (int rr = 0; rr < 4; rr++) {
-    const int br = g * 4 + rr, r = r0 + br;
-    const float v = (float)acc[rr];
-    const bool ok = live_tile && r < R && o < valid_rows;
-    if (kEpi == kQ35Argmax) {
-      keys[br][wave * 16 + o16] = ok ? argmax_key(v, o) : 0ull;
-      if (ok && out) out[(size_t)r * ldo + o] = v;
-    } else if (ok) {
-      float *p = out + (size_t)r * ldo + o;
-      *p = kEpi == kQ35Residual ? *p + v : v;
-    }
-    if (ok && !finitef(v)) atomicOr(&row_err[err_row ? err_row[r] : r], kErrNonFinite);
-  }
-  if (kEpi == kQ35Argmax) {
-    __syncthreads();
-    if (threadIdx.x < kMvRows && r0 + (int)threadIdx.x < R) {
-      unsigned long long best = 0;
-      for (int i = 0; i < 64; i++) best = keys[threadIdx.x][i] > best ? keys[threadIdx.x][i] : best;
-      part[(size_t)(r0 + threadIdx.x) * gridDim.x + blockIdx.x] = best;
-    }
-  }
-}
-
-// The same product for a few rows (decode steps): a workgroup of kWaves
-// waves owns one tile of 16 outputs x 4*kWaves rows, a wave 4 rows, a lane
-// one (output, row) chain, so a 1024-output matrix still spreads over 256
-// waves.  The tile's weights and the rows' activations pass through LDS in
-// chunks of kChunk inputs, double buffered: each thread holds its share of
-// the next chunk in registers while the current chunk is summed, so a whole
-// chunk of work covers the memory latency.  The weights are widened to f32
-// once, when stored to LDS, rather than by each of the 16 lanes that use
-// them.  The k order of each chain is the reference's.
-// kEpi == kQ35Swiglu: eight waves over the same 16 rows, waves 0-3 on gate
-// tile blockIdx.x and waves 4-7 on up tile blockIdx.x + up_off / 16 (up_off
-// passed in valid_rows, F in ldo's place as the output count); the up waves
-// hand their sums to the gate waves through LDS, which write
-// h = (g / (1 + exp(-g))) * u (the SwiGLU pass's expression) to out [R][F].
-template <int kEpi, int kChunk, int kWaves>
-__global__ __launch_bounds__(kWaves * 64) void k_q35_mvd(
-    const uint16_t *__restrict__ w, int valid_rows, int K, const float *__restrict__ x, int ldx,
-    int R, float *out, int ldo, unsigned long long *__restrict__ part, uint32_t *row_err,
-    const uint32_t *__restrict__ err_row) {
+template <int kEpi, int kR, int kW, bool kTail>
+__global__ __launch_bounds__(64 * kW) void k_q35_mv(const uint16_t *__restrict__ w, int valid_rows, int K,
+                                                    const float *__restrict__ x, int ldx, int R, float *out, int ldo,
+                                                    unsigned long long *__restrict__ part, uint32_t *row_err,
+                                                    const uint32_t *__restrict__ err_row) {
   constexpr bool kGlu = kEpi == kQ35Swiglu;
-  constexpr int kTiles = kGlu ? 2 : 1;          // weight tiles per workgroup
-  constexpr int kT = kWaves * 64, kRows = 4 * kWaves / kTiles;
-  constexpr int kXld = kChunk + 4;            // padded LDS row (floats)
-  constexpr int kW4 = kChunk / 8 * 16;        // uint4 words of one tile's weight chunk
-  constexpr int kX4 = kRows * kChunk / 4;     // float4 words of an activation chunk
-  static_assert((kTiles * kW4) % kT == 0 && kX4 % kT == 0, "chunk must split evenly over the threads");
-  __shared__ __align__(16) float4 ws[2][kTiles * 2 * kW4];  // f32 weights [tile][k8][half][output]
-  __shared__ __align__(16) float xs[2][kRows * kXld];
-  const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
-  const int sel = wave / (kWaves / kTiles), wv = wave % (kWaves / kTiles);
-  const int o16 = lane % 16, tile = blockIdx.x, r0 = blockIdx.y * kRows;
-  const int br = wv * 4 + lane / 16, r = r0 + br;
-  const int o = tile * 16 + o16;
-  const bool live = r < R;
-  const int nk8 = K / 8;
-  const uint4 *wt = reinterpret_cast<const uint4 *>(w) + (size_t)tile * nk8 * 16;
-  const uint4 *wt_up = reinterpret_cast<const uint4 *>(w) + (size_t)(tile + (kGlu ? valid_rows / 16 : 0)) * nk8 * 16;
-  uint4 wr[kTiles * kW4 / kT];
-  float4 xr[kX4 / kT];
-  auto fetch = [&](int k0) {
-    const int kc = min(kChunk, K - k0);
-    const int n4 = kc / 8 * 16;  // weight words in this chunk
+  constexpr int kTiles = kGlu ? 2 : 1;
+  __shared__ double s_sum[kW][kTiles][kR][kWave];
+  static_assert(sizeof(float) * kR * kWave <= sizeof(s_sum[0]), "the wave's input strip");
+  const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  float *strip = reinterpret_cast<float *>(s_sum[wave]);  // [kR][64], until the sums take its place
+  const int o16 = lane % 16, koff = 16 * (lane / 16);
+  const int tile = blockIdx.x, r0 = blockIdx.y * kR, nc = (K + 63) / 64;
+  const u32x4q *wt[kTiles];
+  wt[0] = reinterpret_cast<const u32x4q *>(w) + (size_t)tile * (K / 8) * 16 + o16;
+  if constexpr (kGlu) wt[1] = wt[0] + (size_t)(valid_rows / 16) * (K / 8) * 16;
+  const float *xr[kR];
 #pragma unroll
-    for (int i = 0; i < kTiles * kW4 / kT; i++) {
-      const int idx = (tid + kT * i) % kW4;
-      const uint4 *src = (tid + kT * i) < kW4 ? wt : wt_up;
-      wr[i] = idx < n4 ? src[(size_t)k0 / 8 * 16 + idx] : make_uint4(0, 0, 0, 0);
-    }
+  for (int r = 0; r < kR; r++) xr[r] = x + (size_t)min(r0 + r, R - 1) * ldx;  // rows past R: unused
+  double acc[kTiles][kR];
 #pragma unroll
-    for (int i = 0; i < kX4 / kT; i++) {
-      const int idx = tid + kT * i, row = idx / (kChunk / 4), c = (idx % (kChunk / 4)) * 4;
-      xr[i] = (r0 + row < R && c < kc)
-                  ? *reinterpret_cast<const float4 *>(x + (size_t)(r0 + row) * ldx + k0 + c)
-                  : make_float4(0.f, 0.f, 0.f, 0.f);
+  for (int m = 0; m < kTiles; m++)
+#pragma unroll
+    for (int r = 0; r < kR; r++) acc[m][r] = -0.0;
+  struct Step {
+    u32x4q w[kTiles][2];
+    float x[kR];
+  };
+  // branch-free: chunks past the last load it again (unused); inputs past K
+  // (kTail: K not a multiple of 64) become weight +0 and input -0, whose
+  // product -0 changes no sum
+  auto load = [&](Step &st, int c) {
+    const int k = 64 * min(c, nc - 1) + koff;
+#pragma unroll
+    for (int m = 0; m < kTiles; m++)
+#pragma unroll
+      for (int i = 0; i < 2; i++) {
+        const bool in = !kTail || k + 8 * i < K;
+        st.w[m][i] = wt[m][(size_t)(in ? k / 8 + i : 0) * 16];
+        if (!in) st.w[m][i] = u32x4q{0u, 0u, 0u, 0u};
+      }
+#pragma unroll
+    for (int r = 0; r < kR; r++) {
+      const int kx = 64 * min(c, nc - 1) + lane;
+      const bool in = !kTail || kx < K;
+      st.x[r] = xr[r][in ? kx : 0];
+      if (!in) st.x[r] = -0.0f;
     }
   };
-  auto stash = [&](int buf) {
+  auto use = [&](const Step &st) {
 #pragma unroll
-    for (int i = 0; i < kTiles * kW4 / kT; i++) {
-      const int idx = tid + kT * i, t2 = idx / kW4, k8 = idx % kW4 / 16, oo = idx % 16;
-      const uint4 v = wr[i];
-      float4 *dst = ws[buf] + t2 * 2 * kW4;
-      dst[(2 * k8) * 16 + oo] = make_float4(bf_lo(v.x), bf_hi(v.x), bf_lo(v.y), bf_hi(v.y));
-      dst[(2 * k8 + 1) * 16 + oo] = make_float4(bf_lo(v.z), bf_hi(v.z), bf_lo(v.w), bf_hi(v.w));
-    }
+    for (int r = 0; r < kR; r++) strip[r * kWave + lane] = st.x[r];
+    constexpr int kG = kR < 8 ? kR : 8;
 #pragma unroll
-    for (int i = 0; i < kX4 / kT; i++) {
-      const int idx = tid + kT * i, row = idx / (kChunk / 4), c = (idx % (kChunk / 4)) * 4;
-      *reinterpret_cast<float4 *>(&xs[buf][row * kXld + c]) = xr[i];
-    }
-  };
-  fetch(0);
-  stash(0);
-  __syncthreads();
-  double acc = -0.0;
-  int buf = 0;
-  for (int k0 = 0; k0 < K; k0 += kChunk) {
-    const bool more = k0 + kChunk < K;
-    if (more) fetch(k0 + kChunk);
-    const int n8 = min(kChunk, K - k0) / 8;
-    const float4 *wl = ws[buf] + sel * 2 * kW4 + o16;
-    const float *xl = xs[buf] + br * kXld;
-    for (int k8 = 0; k8 < n8; k8++) {
-      const float4 a = wl[(2 * k8) * 16], b = wl[(2 * k8 + 1) * 16];
-      const float4 p = *reinterpret_cast<const float4 *>(xl + k8 * 8);
-      const float4 q = *reinterpret_cast<const float4 *>(xl + k8 * 8 + 4);
-      acc += (double)(a.x * p.x);
-      acc += (double)(a.y * p.y);
-      acc += (double)(a.z * p.z);
-      acc += (double)(a.w * p.w);
-      acc += (double)(b.x * q.x);
-      acc += (double)(b.y * q.y);
-      acc += (double)(b.z * q.z);
-      acc += (double)(b.w * q.w);
-    }
-    if (more) stash(buf ^ 1);
-    __syncthreads();
-    buf ^= 1;
-  }
-  const float v = (float)acc;
-  if constexpr (kGlu) {
-    __shared__ float s_up[kRows][16];
-    const bool ok = live && o < ldo;  // ldo: the output count F
-    if (sel == 1) s_up[br][o16] = v;
-    __syncthreads();
-    if (sel == 0 && ok) {
-      const float u = s_up[br][o16];
-      out[(size_t)r * ldo + o] = (v / (1.0f + exp_f32(-v))) * u;
-    }
-    if (ok && !finitef(v)) atomicOr(&row_err[r], kErrNonFinite);
-    return;
-  }
-  const bool ok = live && o < valid_rows;
-  if (kEpi == kQ35Argmax) {
-    unsigned long long key = ok ? argmax_key(v, o) : 0ull;
+    for (int q = 0; q < 4; q++) {  // inputs 4 q .. + 3 of the lane's 16
+      float wf[kTiles][4];
 #pragma unroll
-    for (int m = 8; m >= 1; m >>= 1) {
-      const unsigned long long other = __shfl_xor(key, m, 16);
-      key = other > key ? other : key;
-    }
-    if (ok && out) out[(size_t)r * ldo + o] = v;
-    if (live && o16 == 0) part[(size_t)r * gridDim.x + tile] = key;
-  } else if (ok) {
-    float *p = out + (size_t)r * ldo + o;
-    *p = kEpi == kQ35Residual ? *p + v : v;
-  }
-  if (ok && !finitef(v)) atomicOr(&row_err[err_row ? err_row[r] : r], kErrNonFinite);
-}
-
-// Broadcast lane J of each 16-lane row to the whole row; folded into the
-// consuming multiply as a DPP operand (row_newbcast).
-template <int J>
-__device__ __forceinline__ float row_bcast(float v) {
-  return __builtin_bit_cast(
-      float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x150 + J, 0xf, 0xf, false));
-}
-
-// Few-rows product split between waves: one wave issues at most one
-// vector instruction every few clocks, so a lane that forms, widens and adds
-// its own products runs its chain at a quarter of the SIMD's pace.  Here the
-// consumer wave (wave 0) owns 64 chains, 16 outputs (lane % 16) x 4 rows
-// (lane / 16), and only adds: per chunk of 16 * kProducers inputs it reads its
-// widened products from LDS, two per read, in k order.  Producer waves
-// 1..kProducers each form 16 of the chunk's products per chain (f32 product,
-// widened to f64) for the next chunk, taking the activation for input j from
-// lane j of the 16-lane row and the weights from registers loaded kDepth
-// chunks ahead.  The consumer's adds are the reference's chain exactly.
-// K % 16 == 0.
-template <int kEpi, int kDepth, int kProducers = 4, int kConsumers = 1>
-__global__ __launch_bounds__(64 * (kProducers + kConsumers)) void k_q35_mvpc(
-    const uint16_t *__restrict__ w, int valid_rows, int K, const float *__restrict__ x, int ldx,
-    int R, float *out, int ldo, unsigned long long *__restrict__ part, uint32_t *row_err,
-    const uint32_t *__restrict__ err_row) {
-  constexpr int kPcChunk = 16 * kProducers;
-  __shared__ __align__(16) double2 pb[2][kPcChunk / 2][64];
-  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-  const int o16 = lane % 16, tile = blockIdx.x;
-  const int r = blockIdx.y * 4 + lane / 16;
-  const int o = tile * 16 + o16;
-  const bool live = r < R;
-  const int nc = (K + kPcChunk - 1) / kPcChunk, ng = K / 16;
-  double acc = -0.0;
-  // consumer wave c (< kConsumers) adds the chains of lanes
-  // [c * 64/kConsumers, (c + 1) * 64/kConsumers); producer p = wave -
-  // kConsumers forms group kProducers * chunk + p of 16 inputs for all 64
-  const bool producer = wave >= kConsumers;
-  const bool mine = !producer && lane / (64 / kConsumers) == wave;
-  const int pg = wave - kConsumers;
-  const uint4 *wt = reinterpret_cast<const uint4 *>(w) + (size_t)tile * (K / 8) * 16 + o16;
-  const float *xr = x + (size_t)(live ? r : 0) * ldx + o16;
-  // two register batches of kDepth chunks each: while one batch is turned
-  // into products, the other is loading (no copies between them, so no load
-  // is waited for before a whole batch of work has passed)
-  float xa[kDepth], xb[kDepth];
-  uint4 wa0[kDepth], wa1[kDepth], wb0[kDepth], wb1[kDepth];
-  auto load = [&](float (&xv)[kDepth], uint4 (&w0)[kDepth], uint4 (&w1)[kDepth], int c0) {
+      for (int m = 0; m < kTiles; m++)
 #pragma unroll
-    for (int j = 0; j < kDepth; j++) {
-      const int g = min(kProducers * (c0 + j) + pg, ng - 1);
-      xv[j] = xr[g * 16];
-      w0[j] = wt[(size_t)(2 * g) * 16];
-      w1[j] = wt[(size_t)(2 * g + 1) * 16];
-    }
-  };
-  auto produce = [&](float xc, uint4 a, uint4 b, int c) {
-    const int g = kProducers * c + pg;
-    if (g >= ng) return;
-    float wf[16] = {bf_lo(a.x), bf_hi(a.x), bf_lo(a.y), bf_hi(a.y), bf_lo(a.z), bf_hi(a.z),
-                    bf_lo(a.w), bf_hi(a.w), bf_lo(b.x), bf_hi(b.x), bf_lo(b.y), bf_hi(b.y),
-                    bf_lo(b.z), bf_hi(b.z), bf_lo(b.w), bf_hi(b.w)};
-    pin_vgprs(wf);
-    float pr[16] = {wf[0] * row_bcast<0>(xc),   wf[1] * row_bcast<1>(xc),
-                    wf[2] * row_bcast<2>(xc),   wf[3] * row_bcast<3>(xc),
-                    wf[4] * row_bcast<4>(xc),   wf[5] * row_bcast<5>(xc),
-                    wf[6] * row_bcast<6>(xc),   wf[7] * row_bcast<7>(xc),
-                    wf[8] * row_bcast<8>(xc),   wf[9] * row_bcast<9>(xc),
-                    wf[10] * row_bcast<10>(xc), wf[11] * row_bcast<11>(xc),
-                    wf[12] * row_bcast<12>(xc), wf[13] * row_bcast<13>(xc),
-                    wf[14] * row_bcast<14>(xc), wf[15] * row_bcast<15>(xc)};
-    double2 *dst = &pb[c & 1][pg * 8][lane];
+        for (int i = 0; i < 2; i++) {
+          wf[m][2 * i] = bf_lo(st.w[m][q / 2][q % 2 * 2 + i]);
+          wf[m][2 * i + 1] = bf_hi(st.w[m][q / 2][q % 2 * 2 + i]);
+        }
 #pragma unroll
-    for (int e = 0; e < 8; e++) dst[e * 64] = make_double2((double)pr[2 * e], (double)pr[2 * e + 1]);
-  };
-  auto consume = [&](int c) {  // chunk c is full (not the last)
-    const double2 *src = &pb[c & 1][0][lane];
+      for (int g = 0; g < kR; g += kG) {
+        float4 xv[kG];
 #pragma unroll
-    for (int e0 = 0; e0 < kPcChunk / 2; e0 += 16) {
-      double2 d[16];
+        for (int r = 0; r < kG; r++) xv[r] = *reinterpret_cast<const float4 *>(strip + (g + r) * kWave + koff + 4 * q);
 #pragma unroll
-      for (int e = 0; e < 16; e++) d[e] = src[(e0 + e) * 64];
+        for (int e = 0; e < 4; e++)
 #pragma unroll
-      for (int e = 0; e < 16; e++) {
-        acc += d[e].x;
-        acc += d[e].y;
+          for (int m = 0; m < kTiles; m++) {
+            float pr[kG];
+            double wd[kG];
+#pragma unroll
+            for (int r = 0; r < kG; r++)
+              pr[r] = wf[m][e] * (e == 0 ? xv[r].x : e == 1 ? xv[r].y : e == 2 ? xv[r].z : xv[r].w);
+            pin_vgprs(pr);
+#pragma unroll
+            for (int r = 0; r < kG; r++) wd[r] = (double)pr[r];
+            pin_vgprs(wd);
+#pragma unroll
+            for (int r = 0; r < kG; r++) acc[m][g + r] += wd[r];
+          }
       }
     }
   };
-  if (producer) load(xa, wa0, wa1, 0);
-  // whole turns of 2*kDepth chunks; steps past the last chunk only keep the
-  // barrier count uniform.  Step c: producers fill chunk c, the consumer adds
-  // chunk c-1.
-  const int ncp = (nc + 2 * kDepth - 1) / (2 * kDepth) * (2 * kDepth);
-  for (int c0 = 0; c0 < ncp; c0 += 2 * kDepth) {
-    if (producer) load(xb, wb0, wb1, c0 + kDepth);
-#pragma unroll
-    for (int j = 0; j < kDepth; j++) {
-      const int c = c0 + j;
-      if (producer) produce(xa[j], wa0[j], wa1[j], c);
-      else if (mine && c > 0 && c < nc) consume(c - 1);
-      __syncthreads();
-    }
-    if (producer) load(xa, wa0, wa1, c0 + 2 * kDepth);
-#pragma unroll
-    for (int j = 0; j < kDepth; j++) {
-      const int c = c0 + kDepth + j;
-      if (producer) produce(xb[j], wb0[j], wb1[j], c);
-      else if (mine && c > 0 && c < nc) consume(c - 1);
-      __syncthreads();
+  Step a, b;  // two register sets, one loading while the other is used
+  load(a, wave);
+  for (int c = wave; c < nc; c += 2 * kW) {
+    load(b, c + kW);
+    use(a);
+    if (c + kW < nc) {
+      load(a, c + 2 * kW);
+      use(b);
     }
   }
-  if (!mine) return;
-  {
-    const int c = nc - 1;
-    const int n2 = min(kPcChunk, K - c * kPcChunk) / 2;
-    const double2 *src = &pb[c & 1][0][lane];
-    for (int e = 0; e < n2; e++) {
-      const double2 d = src[e * 64];
-      acc += d.x;
-      acc += d.y;
-    }
-  }
-  const float v = (float)acc;
-  const bool ok = live && o < valid_rows;
-  if (kEpi == kQ35Argmax) {
-    unsigned long long key = ok ? argmax_key(v, o) : 0ull;
+  // (each wave's sums take its own strip's place: its reads are behind it)
 #pragma unroll
-    for (int m = 8; m >= 1; m >>= 1) {
-      const unsigned long long other = __shfl_xor(key, m, 16);
-      key = other > key ? other : key;
+  for (int m = 0; m < kTiles; m++)
+#pragma unroll
+    for (int r = 0; r < kR; r++) s_sum[wave][m][r][lane] = acc[m][r];
+  __syncthreads();
+  for (int idx = threadIdx.x; idx < kR * 16; idx += 64 * kW) {
+    const int br = idx / 16, oo = idx % 16, r = r0 + br, o = tile * 16 + oo;
+    float v[kTiles];
+#pragma unroll
+    for (int m = 0; m < kTiles; m++) {
+      double sum = -0.0;
+#pragma unroll
+      for (int i = 0; i < kW; i++)
+#pragma unroll
+        for (int q = 0; q < 4; q++) sum += s_sum[i][m][br][q * 16 + oo];
+      v[m] = (float)sum;
     }
-    if (ok && out) out[(size_t)r * ldo + o] = v;
-    if (live && o16 == 0) part[(size_t)r * gridDim.x + tile] = key;
-  } else if (ok) {
-    float *p = out + (size_t)r * ldo + o;
-    *p = kEpi == kQ35Residual ? *p + v : v;
+    bool bad = !finitef(v[0]);
+    if constexpr (kGlu) {
+      const bool ok = r < R && o < ldo;  // ldo: the output count F
+      bad |= !finitef(v[kTiles - 1]);
+      if (ok) out[(size_t)r * ldo + o] = (v[0] / (1.0f + exp_f32(-v[0]))) * v[kTiles - 1];
+      if (ok && bad) atomicOr(&row_err[r], kErrNonFinite);
+    } else {
+      const bool ok = r < R && o < valid_rows;
+      if constexpr (kEpi == kQ35Argmax) {
+        unsigned long long key = ok ? argmax_key(v[0], o) : 0ull;
+#pragma unroll
+        for (int m = 8; m >= 1; m >>= 1) {
+          const unsigned long long other = __shfl_xor(key, m, 16);
+          key = other > key ? other : key;
+        }
+        if (ok && out) out[(size_t)r * ldo + o] = v[0];
+        if (r < R && oo == 0) part[(size_t)r * gridDim.x + tile] = key;
+      } else if (ok) {
+        float *p = out + (size_t)r * ldo + o;
+        *p = kEpi == kQ35Residual ? *p + v[0] : v[0];
+      }
+      if (ok && bad) atomicOr(&row_err[err_row ? err_row[r] : r], kErrNonFinite);
+    }
   }
-  if (ok && !finitef(v)) atomicOr(&row_err[err_row ? err_row[r] : r], kErrNonFinite);
 }
 
 // cpu.rs:74-78 swiglu
@@ -1296,53 +1108,52 @@ void q35_norm(hipStream_t s, int rows, const float *x, int ldx, const uint32_t *
 
 int q35_matvec_blocks(int rows_w) { return (rows_w + 15) / 16; }
 
-// Up to this many rows the one-chain-per-lane form runs (and always for the
-// argmax head, whose partials are per 16-output tile).
-constexpr int kMvdMaxRows = 64;
+// Rows per workgroup (kR) and waves that split K (kW).  More rows share each
+// weight load and widening, but the grid has to fill the CUs: at 16 rows o and
+// down (64 tiles) take 7.3 and 10.0 us as four rows on eight waves, 10.0 and
+// 14.6 as eight; gate+up (224 pairs) 15.0 as eight rows on four waves, 15.2 as
+// four, 18.9 as sixteen; mix (514 tiles) 17.1, 17.2 and 20.1; the head (15,520
+// tiles) 340 as sixteen, 346 as eight, 399 as four.
+template <int kEpi>
+static void mv(hipStream_t s, const uint16_t *w, int tiles, int valid_rows, int K, const float *x, int ldx, int R,
+               float *out, int ldo, unsigned long long *part, uint32_t *row_err, const uint32_t *err_row) {
+  auto go = [&](auto kr, auto kw) {
+    constexpr int kR = decltype(kr)::value, kW = decltype(kw)::value;
+    const dim3 grid(tiles, (R + kR - 1) / kR);
+    if (K % 64 == 0)
+      hipLaunchKernelGGL((k_q35_mv<kEpi, kR, kW, false>), grid, dim3(64 * kW), 0, s, w, valid_rows, K, x, ldx, R, out,
+                         ldo, part, row_err, err_row);
+    else
+      hipLaunchKernelGGL((k_q35_mv<kEpi, kR, kW, true>), grid, dim3(64 * kW), 0, s, w, valid_rows, K, x, ldx, R, out,
+                         ldo, part, row_err, err_row);
+  };
+  using std::integral_constant;
+  const int g8 = tiles * ((R + 7) / 8), g4 = tiles * ((R + 3) / 4);
+  if (R > 8 && tiles * ((R + 15) / 16) >= 4096)
+    go(integral_constant<int, 16>{}, integral_constant<int, 4>{});
+  else if (R > 4 && g8 >= 448)
+    go(integral_constant<int, 8>{}, integral_constant<int, 4>{});
+  else if (g4 >= 448)
+    go(integral_constant<int, 4>{}, integral_constant<int, 4>{});
+  else
+    go(integral_constant<int, 4>{}, integral_constant<int, 8>{});
+}
 
 void q35_matvec(hipStream_t s, int epi, const uint16_t *w, int rows_w, int valid_rows, int K,
                 const float *x, int ldx, int R, float *out, int ldo, unsigned long long *part,
                 uint32_t *row_err, const uint32_t *err_row) {
-  if (R <= kMvdMaxRows || epi == kQ35Argmax) {
-    const int tiles = rows_w / 16;
-    // Few (16-output tile, 4-row group) pairs: one chain per lane leaves most
-    // SIMDs with a single wave, so the chains' adds go to consumer waves fed
-    // by producer waves.  Otherwise the one-wave-per-chain-set form, four
-    // waves per workgroup, three workgroups per CU.
-    if (epi != kQ35Argmax && K % 16 == 0 && tiles * ((R + 3) / 4) <= 512) {
-      const dim3 grid(tiles, (R + 3) / 4);
-      // eight producers (128-input chunks, 128 KB of LDS, one workgroup per
-      // CU) against four: C5 one-token steps 3.76 -> 3.65 ms
-      if (epi == kQ35Store)
-        hipLaunchKernelGGL((k_q35_mvpc<kQ35Store, 2, 8, 1>), grid, dim3(576), 0, s, w, valid_rows,
-                           K, x, ldx, R, out, ldo, part, row_err, err_row);
-      else
-        hipLaunchKernelGGL((k_q35_mvpc<kQ35Residual, 2, 8, 1>), grid, dim3(576), 0, s, w,
-                           valid_rows, K, x, ldx, R, out, ldo, part, row_err, err_row);
-      return;
-    }
-    const dim3 grid(tiles, (R + 15) / 16);
-    if (epi == kQ35Store)
-      hipLaunchKernelGGL((k_q35_mvd<kQ35Store, 128, 4>), grid, dim3(256), 0, s, w, valid_rows, K, x,
-                         ldx, R, out, ldo, part, row_err, err_row);
-    else if (epi == kQ35Residual)
-      hipLaunchKernelGGL((k_q35_mvd<kQ35Residual, 128, 4>), grid, dim3(256), 0, s, w, valid_rows,
-                         K, x, ldx, R, out, ldo, part, row_err, err_row);
-    else
-      hipLaunchKernelGGL((k_q35_mvd<kQ35Argmax, 128, 4>), grid, dim3(256), 0, s, w, valid_rows, K,
-                         x, ldx, R, out, ldo, part, row_err, err_row);
-    return;
-  }
-  const dim3 grid((rows_w + 63) / 64, (R + kMvRows - 1) / kMvRows);
+  const int tiles = rows_w / 16;
   if (epi == kQ35Store)
-    hipLaunchKernelGGL(k_q35_mv<kQ35Store>, grid, dim3(256), 0, s, w, rows_w, valid_rows, K, x,
-                       ldx, R, out, ldo, part, row_err, err_row);
+    mv<kQ35Store>(s, w, tiles, valid_rows, K, x, ldx, R, out, ldo, part, row_err, err_row);
   else if (epi == kQ35Residual)
-    hipLaunchKernelGGL(k_q35_mv<kQ35Residual>, grid, dim3(256), 0, s, w, rows_w, valid_rows, K,
-                       x, ldx, R, out, ldo, part, row_err, err_row);
+    mv<kQ35Residual>(s, w, tiles, valid_rows, K, x, ldx, R, out, ldo, part, row_err, err_row);
   else
-    hipLaunchKernelGGL(k_q35_mv<kQ35Argmax>, grid, dim3(256), 0, s, w, rows_w, valid_rows, K, x,
-                       ldx, R, out, ldo, part, row_err, err_row);
+    mv<kQ35Argmax>(s, w, tiles, valid_rows, K, x, ldx, R, out, ldo, part, row_err, err_row);
+}
+
+void q35_matvec_swiglu(hipStream_t s, const uint16_t *w, int up_off, int F, int K, const float *x,
+                       int ldx, int R, float *h, uint32_t *row_err) {
+  mv<kQ35Swiglu>(s, w, up_off / 16, up_off, K, x, ldx, R, h, F, nullptr, row_err, nullptr);
 }
 
 void q35_split_bf16(hipStream_t s, int rows, int K, const float *x, int ldx, uint16_t *hi, uint16_t *lo) {
@@ -1375,17 +1186,6 @@ void q35_gemm_split(hipStream_t s, bool accumulate, const uint16_t *w, int N, in
     hipLaunchKernelGGL((k_gemm<kBF16, true, 2, 4, 4, 2, 2, kAccumulate>), grid, dim3(512), lds, s, g);
   else
     hipLaunchKernelGGL((k_gemm<kBF16, true, 2, 4, 4, 2, 2, kStore>), grid, dim3(512), lds, s, g);
-}
-
-bool q35_matvec_swiglu(hipStream_t s, const uint16_t *w, int up_off, int F, int K, const float *x,
-                       int ldx, int R, float *h, int ldh, uint32_t *row_err) {
-  const int tiles = 2 * up_off / 16;  // gate and up tiles, as q35_matvec sees the matrix
-  if (R > kMvdMaxRows || up_off % 16 || K % 8 || ldh != F ||
-      (K % 16 == 0 && tiles * ((R + 3) / 4) <= 512))
-    return false;
-  hipLaunchKernelGGL((k_q35_mvd<kQ35Swiglu, 128, 8>), dim3(up_off / 16, (R + 15) / 16), dim3(512), 0,
-                     s, w, up_off, K, x, ldx, R, h, F, nullptr, row_err, nullptr);
-  return true;
 }
 
 void q35_swiglu(hipStream_t s, int rows, const float *gu, int ldgu, int F, int up_off, float *h,
