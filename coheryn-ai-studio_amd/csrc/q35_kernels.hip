@@ -34,9 +34,13 @@ __device__ __forceinline__ float sigmoid_f32(float x) {
 }
 __device__ __forceinline__ float silu_f32(float x) { return x * sigmoid_f32(x); }
 // The same with expf's table staged in LDS (per-lane reads).
-__device__ __forceinline__ float silu_f32(float x, const uint64_t *tab) {
+__device__ __forceinline__ float sigmoid_f32(float x, const uint64_t *tab) {
   const float e = exp_f32_tab(-fabsf(x), tab);
-  return x * (x >= 0.0f ? 1.0f / (1.0f + e) : e / (1.0f + e));
+  return x >= 0.0f ? 1.0f / (1.0f + e) : e / (1.0f + e);
+}
+__device__ __forceinline__ float silu_f32(float x, const uint64_t *tab) { return x * sigmoid_f32(x, tab); }
+__device__ __forceinline__ float softplus_f32(float x, const uint64_t *tab) {
+  return fmaxf(x, 0.0f) + log1p_f32(exp_f32_tab(-fabsf(x), tab));
 }
 __device__ __forceinline__ float softplus_f32(float x) {
   return fmaxf(x, 0.0f) + log1p_f32(exp_f32(-fabsf(x)));
@@ -51,30 +55,6 @@ __global__ __launch_bounds__(256) void k_q35_embed(const uint16_t *__restrict__ 
   const int r = blockIdx.x;
   const uint16_t *src = embed + (size_t)tokens[r] * H;
   for (int i = threadIdx.x; i < H; i += 256) x[(size_t)r * H + i] = bf_lo(src[i]);
-}
-
-// Sum of v[0..n) in f64, in index order from `init`, by one lane: the
-// terms stream from LDS in batches of 16, the next batch loading while the
-// current one is added, so the dependent add chain sets the pace.
-__device__ __forceinline__ double ordered_sum_f64(const double *v, int n, double init) {
-  double sum = init;
-  const int n16 = n / 16;
-  double cur[16], nxt[16];
-  if (n16) {
-#pragma unroll
-    for (int j = 0; j < 16; j++) cur[j] = v[j];
-  }
-  for (int b = 0; b < n16; b++) {
-    const int nb = min(b + 1, n16 - 1) * 16;
-#pragma unroll
-    for (int j = 0; j < 16; j++) nxt[j] = v[nb + j];
-#pragma unroll
-    for (int j = 0; j < 16; j++) sum += cur[j];
-#pragma unroll
-    for (int j = 0; j < 16; j++) cur[j] = nxt[j];
-  }
-  for (int i = n16 * 16; i < n; i++) sum += v[i];
-  return sum;
 }
 
 // ---------------------------------------------------------------------------
@@ -598,9 +578,13 @@ __global__ __launch_bounds__(256) void k_q35_delta(Q35Lanes L, const float *__re
 // workgroup, token after token (execution.rs:357-411): the causal conv of the
 // head's q, k (its key head's channels) and v channels, the q/k norms and
 // gates, the delta-rule column updates, and the output norm times SiLU(z).
-// Thread j owns q/k channel j of the key head (j < kKD), v channel and state
-// column j of the value head (j < VD).  The arithmetic of each stage is the
-// one the separate kernels above restate; only the launches are merged.
+// kP lanes own one state column, kKD / kP keys each, as in k_q35_delta, and
+// every sum is a fixed tree as in the separate kernels; the arithmetic of each
+// stage is theirs.  (One thread per column with ordered sums took 19 us a
+// launch at 16 one-token lanes x 16 heads, most of it waiting on one lane's
+// adds; this takes 15.  Whole waves hold one part of the columns, so the state
+// streams in 256-byte rows and the partial sums meet in LDS: with the lanes of
+// a column side by side, in 32-byte pieces and DPP sums, it took 18.)
 // Used when every value head has its own key head: a workgroup then owns all
 // the conv channels it reads and writes back (with shared key heads the ring
 // would be read by one workgroup after another had advanced it).  Conv
@@ -618,7 +602,7 @@ __device__ __forceinline__ void conv_load(ConvTaps &c, const float *h, const flo
     c.w[i] = i < K ? w[i] : 0.0f;
   }
 }
-__device__ __forceinline__ float conv_step(ConvTaps &c, float in, int K) {
+__device__ __forceinline__ float conv_step(ConvTaps &c, float in, int K, const uint64_t *tab) {
 #pragma unroll
   for (int i = 0; i < kFusedConv - 1; i++)
     if (i < K - 1) c.tap[i] = c.tap[i + 1];
@@ -629,7 +613,7 @@ __device__ __forceinline__ float conv_step(ConvTaps &c, float in, int K) {
 #pragma unroll
   for (int i = 0; i < kFusedConv; i++)
     if (i < K) sum += (double)(c.tap[i] * c.w[i]);
-  return silu_f32((float)sum);
+  return silu_f32((float)sum, tab);
 }
 __device__ __forceinline__ void conv_store(const ConvTaps &c, float *h, int K, int c1) {
 #pragma unroll
@@ -637,180 +621,165 @@ __device__ __forceinline__ void conv_store(const ConvTaps &c, float *h, int K, i
     if (i < K) h[(c1 + i) % K] = c.tap[i];
 }
 
-template <int kKD>
-__global__ __launch_bounds__(256) void k_q35_linear(
+template <int kKD, int kP>
+__global__ __launch_bounds__(1024) void k_q35_linear(
     Q35Lanes L, const float *__restrict__ mix, int ldm, int keys, int z_off, int a_off, int b_off,
     const float *__restrict__ conv_w, int K, float *hist, size_t hist_seq,
     const float *__restrict__ a_log, const float *__restrict__ dt,
     const float *__restrict__ norm_w, int KH, int VH, int VD, float eps, float *state,
     size_t state_seq, float *__restrict__ tgt, int ldt, uint32_t *row_err) {
-  __shared__ __align__(16) float qv[kKD], kv[kKD], s_qq[kKD], s_kk[kKD];
-  __shared__ double qsq[kKD], ksq[kKD], osq[256];
-  __shared__ float s_qn, s_kn, s_scale;
-  __shared__ float4 s_gate;
+  constexpr int kCells = kKD / kP;                // keys per thread
+  constexpr int kN = kKD < kWave ? kKD : kWave;   // channels of one norm partial
+  __shared__ __align__(16) float s_q[kKD], s_k[kKD], s_v[256];
+  __shared__ double s_p[2][1024];
+  __shared__ double s_sq[1024 / kN], s_o[1024 / kWave];
+  __shared__ float s_decay, s_beta;
   __shared__ int s_bad;
-  const int ln = blockIdx.x, h = blockIdx.y, j = threadIdx.x;
+  __shared__ uint64_t s_tab[32];
+  const int ln = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
+  if (tid < 32) s_tab[tid] = kExp2Tab[tid];
   const int rep = VH / KH, src = (h / rep) * kKD;
   const uint32_t first = L.first[ln], n = L.n[ln], start = L.start[ln];
   const uint32_t seq = L.seq[ln];
-  const bool has_qk = j < kKD, has_v = j < VD;
   float *hs = hist + (size_t)seq * hist_seq;
   const int c0 = (int)(start % (uint32_t)K);
-  const int qc = src + j, kc = keys + src + j, vc = 2 * keys + h * VD + j;
-  ConvTaps cq, ck, cv;
-  if (has_qk) {
-    conv_load(cq, hs + (size_t)qc * K, conv_w + (size_t)qc * K, K, c0);
-    conv_load(ck, hs + (size_t)kc * K, conv_w + (size_t)kc * K, K, c0);
-  }
-  if (has_v) conv_load(cv, hs + (size_t)vc * K, conv_w + (size_t)vc * K, K, c0);
-  float *S = state + (size_t)seq * state_seq + (size_t)h * kKD * VD;
-  const __amdgpu_buffer_rsrc_t rs =
-      __builtin_amdgcn_make_buffer_rsrc(S, (short)0, (int)(kKD * VD * 4), 0x00020000);
-  const int voff = has_v ? j * 4 : 0;
-  float col[kKD];
+  // conv roles: thread tid brings q channel tid, k channel tid - kKD or v
+  // channel tid - 2 kKD (the launch gives at least 2 kKD + VD threads)
+  const bool has_c = tid < 2 * kKD + VD;
+  const int ch = tid < kKD ? src + tid : tid < 2 * kKD ? keys + src + tid - kKD : 2 * keys + h * VD + tid - 2 * kKD;
+  // the first token's small inputs are requested before the state: loads
+  // complete in order, and the conv and the gate then run under the state's
+  ConvTaps ct;
+  if (has_c) conv_load(ct, hs + (size_t)ch * K, conv_w + (size_t)ch * K, K, c0);
+  const bool gate = tid == (int)blockDim.x - 1;
+  float in = 0.0f, a_in = 0.0f, b_in = 0.0f;
+  auto small = [&](uint32_t t) {
+    const float *mr = mix + (size_t)(first + t) * ldm;
+    if (has_c) in = mr[ch];
+    if (gate) {
+      a_in = mr[a_off + h];
+      b_in = mr[b_off + h];
+    }
+  };
+  if (n) small(0);
+  const float al = gate ? a_log[h] : 0.0f, dtb = gate ? dt[h] : 0.0f;
+  __builtin_amdgcn_sched_barrier(0);
+  // delta roles: part `part` of state column j
+  // (whole waves of one part, so a wave's state loads are contiguous)
+  const int vdp = (VD + kWave - 1) / kWave * kWave;
+  const int part = __builtin_amdgcn_readfirstlane(tid / vdp), j = tid % vdp;
+  const bool active = j < VD && part < kP;
+  float *S = state + (size_t)seq * state_seq + (size_t)h * kKD * VD + (active ? j : 0);
+  float col[kCells];
 #pragma unroll
-  for (int i = 0; i < kKD; i++)
-    col[i] = has_v ? __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, voff, i * VD * 4, 0))
-                   : 0.0f;
-  const int T = blockDim.x;
-  const float nw = has_v ? norm_w[j] : 0.0f;
+  for (int i = 0; i < kCells; i++) col[i] = active ? S[(size_t)(kCells * part + i) * VD] : 0.0f;
+  const float nw = active ? norm_w[j] : 0.0f;
+  __builtin_amdgcn_sched_barrier(0);
+  __syncthreads();  // s_tab
+  // a column's partial sums meet in LDS and are added in part order
+  auto all_parts = [&](int which, double v) {
+    if constexpr (kP == 1) return v;
+    s_p[which][tid] = v;
+    __syncthreads();
+    double sum = s_p[which][j];
+#pragma unroll
+    for (int i = 1; i < kP; i++) sum += s_p[which][i * vdp + j];
+    return sum;
+  };
   for (uint32_t t = 0; t < n; t++) {
     const uint32_t row = first + t;
     const float *mr = mix + (size_t)row * ldm;
+    const float z = active ? mr[z_off + h * VD + j] : 0.0f;
     bool bad = false;
     // causal conv + SiLU (kernels.rs:54-120)
-    if (has_qk) {
-      const float iq = mr[qc], ik = mr[kc];
-      const float q = conv_step(cq, iq, K), k = conv_step(ck, ik, K);
-      qv[j] = q;
-      kv[j] = k;
-      qsq[j] = (double)(q * q);
-      ksq[j] = (double)(k * k);
-      bad |= !finitef(iq) || !finitef(ik) || !finitef(q) || !finitef(k);
+    float y = 0.0f;
+    if (has_c) {
+      y = conv_step(ct, in, K, s_tab);
+      bad |= !finitef(in) || !finitef(y);
+      if (tid < 2 * kKD) {
+        (tid < kKD ? s_q : s_k)[tid % kKD] = y;
+      } else {
+        s_v[tid - 2 * kKD] = y;
+      }
     }
-    float v = 0.0f;
-    if (has_v) {
-      const float iv = mr[vc];
-      v = conv_step(cv, iv, K);
-      bad |= !finitef(iv) || !finitef(v);
+    // q/k norms: a tree over each kN channels, then (128 keys) two in order
+    double sq = (double)(y * y);
+#pragma unroll
+    for (int m = 1; m < kN; m <<= 1) sq += __shfl_xor(sq, m, kWave);
+    if (tid % kN == 0) s_sq[tid / kN] = sq;
+    if (gate) {
+      const float ld = -exp_f32_tab(al, s_tab) * softplus_f32(a_in + dtb, s_tab);
+      const float beta = sigmoid_f32(b_in, s_tab);
+      s_decay = exp_f32_tab(ld, s_tab);
+      s_beta = beta;
+      s_bad = !finitef(ld) || !finitef(beta) || ld > 0.0f || !(beta >= 0.0f && beta <= 1.0f);
     }
+    if (t + 1 < n) small(t + 1);
     __syncthreads();
-    // q/k norms: ordered f64 sums of the f32 squares, in two waves when there are two
-    if (j == 0) s_qn = (float)ordered_sum_f64(qsq, kKD, -0.0);
-    if (j == (T > kWave ? kWave : 0)) s_kn = (float)ordered_sum_f64(ksq, kKD, -0.0);
-    __syncthreads();
-    if (j == 0) {
-      const float qn = s_qn, kn = s_kn;
-      const float ld = -exp_f32(a_log[h]) * softplus_f32(mr[a_off + h] + dt[h]);
-      const float beta = sigmoid_f32(mr[b_off + h]);
-      s_gate = make_float4((1.0f / sqrtf(qn + 1e-6f)) / sqrtf((float)kKD), 1.0f / sqrtf(kn + 1e-6f),
-                           exp_f32(ld), beta);
-      s_bad = !finitef(qn) || !finitef(kn) || !finitef(ld) || !finitef(beta) || ld > 0.0f ||
-              !(beta >= 0.0f && beta <= 1.0f);
+    constexpr int kNP = kKD / kN;
+    double qs = s_sq[0], ks = s_sq[kNP];
+    if constexpr (kNP == 2) {
+      qs += s_sq[1];
+      ks += s_sq[3];
     }
-    __syncthreads();
-    const float4 gt = s_gate;
-    if (has_qk) {
-      s_qq[j] = qv[j] * gt.x;
-      s_kk[j] = kv[j] * gt.y;
-    }
-    __syncthreads();
-    // the delta rule on state column j (kernels.rs:122-214)
+    const float qn = (float)qs, kn = (float)ks;
+    bad |= !finitef(qn) || !finitef(kn);
+    const float q_scale = (1.0f / sqrtf(qn + 1e-6f)) / sqrtf((float)kKD), k_scale = 1.0f / sqrtf(kn + 1e-6f);
+    // the delta rule on state column j (kernels.rs:122-214), as in k_q35_delta
     float o = 0.0f;
-    if (has_v) {
-      const float decay = gt.z, beta = gt.w;
-      // LDS values two groups of 4 ahead of their use, as in k_q35_delta
-      const float4 *kk4 = reinterpret_cast<const float4 *>(s_kk);
-      const float4 *qq4 = reinterpret_cast<const float4 *>(s_qq);
-      constexpr int kG4 = kKD / 4;
+    {
+      const float decay = s_decay, beta = s_beta, v = s_v[min(j, VD - 1)];
       double pred = 0.0;
-      float4 ka = kk4[0], kb = kG4 > 1 ? kk4[1] : ka;
+      float kk[kCells];
 #pragma unroll
-      for (int i0 = 0; i0 < kKD; i0 += 4) {
-        asm volatile("" ::: "memory");
-        const float4 kq = ka;
-        ka = kb;
-        if (i0 / 4 + 2 < kG4) kb = kk4[i0 / 4 + 2];
-        const float k4[4] = {kq.x, kq.y, kq.z, kq.w};
-        float p[4];
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-          col[i0 + e] *= decay;
-          p[e] = col[i0 + e] * k4[e];
-        }
-        pin_vgprs(p);
-        double wd[4];
-#pragma unroll
-        for (int e = 0; e < 4; e++) wd[e] = (double)p[e];
-        pin_vgprs(wd);
-#pragma unroll
-        for (int e = 0; e < 4; e++) pred += wd[e];
+      for (int u = 0; u < kCells / 4; u++) {
+        const float4 a = *reinterpret_cast<const float4 *>(&s_k[part % kP * kCells + 4 * u]);
+        kk[4 * u] = a.x * k_scale; kk[4 * u + 1] = a.y * k_scale;
+        kk[4 * u + 2] = a.z * k_scale; kk[4 * u + 3] = a.w * k_scale;
       }
-      const float corr = (v - (float)pred) * beta;
+#pragma unroll
+      for (int i = 0; i < kCells; i++) {
+        col[i] *= decay;
+        pred += (double)(col[i] * kk[i]);
+      }
+      const float corr = (v - (float)all_parts(0, pred)) * beta;
       double rd = 0.0;
-      ka = kk4[0];
-      kb = kG4 > 1 ? kk4[1] : ka;
-      float4 qa = qq4[0], qb = kG4 > 1 ? qq4[1] : qa;
 #pragma unroll
-      for (int i0 = 0; i0 < kKD; i0 += 4) {
-        asm volatile("" ::: "memory");
-        const float4 kq = ka, qq = qa;
-        ka = kb;
-        qa = qb;
-        if (i0 / 4 + 2 < kG4) {
-          kb = kk4[i0 / 4 + 2];
-          qb = qq4[i0 / 4 + 2];
-        }
-        const float k4[4] = {kq.x, kq.y, kq.z, kq.w}, q4[4] = {qq.x, qq.y, qq.z, qq.w};
-        float p[4];
+      for (int u = 0; u < kCells / 4; u++) {
+        const float4 a = *reinterpret_cast<const float4 *>(&s_q[part % kP * kCells + 4 * u]);
+        const float qq[4] = {a.x * q_scale, a.y * q_scale, a.z * q_scale, a.w * q_scale};
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-          col[i0 + e] += k4[e] * corr;
-          p[e] = col[i0 + e] * q4[e];
+          col[4 * u + e] += kk[4 * u + e] * corr;
+          rd += (double)(col[4 * u + e] * qq[e]);
         }
-        pin_vgprs(p);
-        double wd[4];
-#pragma unroll
-        for (int e = 0; e < 4; e++) wd[e] = (double)p[e];
-        pin_vgprs(wd);
-#pragma unroll
-        for (int e = 0; e < 4; e++) rd += wd[e];
       }
-      o = (float)rd;
       // a non-finite updated cell makes o non-finite (its read product is
       // inf or NaN, and no f64 sum returns from those), so o covers the cells
-      bad |= !finitef(o);
-      osq[j] = (double)(o * o);
+      o = (float)all_parts(1, rd);
+      bad |= active && !finitef(o);
     }
-    __syncthreads();
     // output norm over the head (zero_centered false) times SiLU(z) (execution.rs:397-411)
-    if (j == 0) {
-      const double sum = ordered_sum_f64(osq, VD, -0.0);
-      const double mean = sum / (double)VD;
-      s_bad |= !(__builtin_isfinite(mean) && finitef((float)mean));
-      s_scale = 1.0f / sqrtf((float)mean + eps);
-    }
+    const double os = wave_sum_f64(active && part == 0 ? (double)(o * o) : -0.0);
+    if (tid % kWave == 0) s_o[tid / kWave] = os;
     __syncthreads();
-    if (has_v) {
-      const float z = mr[z_off + h * VD + j];
-      const float y = ((o * s_scale) * (nw + 0.0f)) * silu_f32(z);
-      tgt[(size_t)row * ldt + h * VD + j] = y;
-      bad |= !finitef(y);
+    double sum = s_o[0];
+    for (int i = 1; i < (int)blockDim.x / kWave; i++) sum += s_o[i];
+    const double mean = sum / (double)VD;
+    bad |= !(__builtin_isfinite(mean) && finitef((float)mean));
+    if (active && part == 0) {
+      const float yo = ((o * (1.0f / sqrtf((float)mean + eps))) * (nw + 0.0f)) * silu_f32(z, s_tab);
+      tgt[(size_t)row * ldt + h * VD + j] = yo;
+      bad |= !finitef(yo);
     }
-    if (bad || (j == 0 && s_bad)) atomicOr(&row_err[row], kErrRequest);
+    if (bad || (tid == 0 && s_bad)) atomicOr(&row_err[row], kErrRequest);
     __syncthreads();  // the LDS stages are rewritten by the next token
   }
   const int c1 = (int)((start + n) % (uint32_t)K);
-  if (has_qk) {
-    conv_store(cq, hs + (size_t)qc * K, K, c1);
-    conv_store(ck, hs + (size_t)kc * K, K, c1);
-  }
-  if (has_v) {
-    conv_store(cv, hs + (size_t)vc * K, K, c1);
+  if (has_c) conv_store(ct, hs + (size_t)ch * K, K, c1);
+  if (active) {
 #pragma unroll
-    for (int i = 0; i < kKD; i++)
-      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, col[i]), rs, voff,
-                                            i * VD * 4, 0);
+    for (int i = 0; i < kCells; i++) S[(size_t)(kCells * part + i) * VD] = col[i];
   }
 }
 
@@ -1213,18 +1182,26 @@ void q35_linear(hipStream_t s, int lanes, Q35Lanes L, const float *mix, int ldm,
                 int key_heads, int value_heads, int key_dim, int value_dim, float eps,
                 float *state, size_t state_seq, float *tgt, int ldt, uint32_t *row_err) {
   const dim3 grid(lanes, value_heads);
-  const dim3 block(((std::max(key_dim, value_dim) + kWave - 1) / kWave) * kWave);
-#define LIN_(KD)                                                                               \
-  case KD:                                                                                     \
-    hipLaunchKernelGGL(k_q35_linear<KD>, grid, block, 0, s, L, mix, ldm, keys, z_off, a_off,  \
-                       b_off, conv_w, K, hist, hist_seq, a_log, dt, norm_w, key_heads,           \
-                       value_heads, value_dim, eps, state, state_seq, tgt, ldt, row_err);      \
-    break;
+  // a column's lanes: 16 keys each, or 32 where 128 keys x more than 128
+  // columns would pass 1,024 threads
+  auto go = [&](auto kd, auto parts) {
+    constexpr int kKD = decltype(kd)::value, kP = decltype(parts)::value;
+    const int vdp = (value_dim + kWave - 1) / kWave * kWave;
+    const int threads = (std::max(vdp * kP, 2 * kKD + value_dim) + kWave - 1) / kWave * kWave;
+    hipLaunchKernelGGL((k_q35_linear<kKD, kP>), grid, dim3(threads), 0, s, L, mix, ldm, keys, z_off, a_off, b_off,
+                       conv_w, K, hist, hist_seq, a_log, dt, norm_w, key_heads, value_heads, value_dim, eps, state,
+                       state_seq, tgt, ldt, row_err);
+  };
+  using std::integral_constant;
   switch (key_dim) {
-    LIN_(16) LIN_(32) LIN_(64) LIN_(128)
-    default: break;
+    case 16: return go(integral_constant<int, 16>{}, integral_constant<int, 1>{});
+    case 32: return go(integral_constant<int, 32>{}, integral_constant<int, 2>{});
+    case 64: return go(integral_constant<int, 64>{}, integral_constant<int, 4>{});
+    case 128:
+      if (value_dim <= 128) return go(integral_constant<int, 128>{}, integral_constant<int, 8>{});
+      return go(integral_constant<int, 128>{}, integral_constant<int, 4>{});
+    default: return;
   }
-#undef LIN_
 }
 
 bool q35_delta_supported(int key_dim, int value_dim) {
