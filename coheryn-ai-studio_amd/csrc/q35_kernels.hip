@@ -937,9 +937,10 @@ __global__ __launch_bounds__(256) void k_q35_scores(Q35Rows Rw, const float *__r
 // exp(s_t - m_t) are formed in parallel from the scores; the two f32
 // recurrences den = den*old + new and o_d = o_d*old + new*v_d then run in key
 // order, one thread per output element (and one for the denominator), V
-// loads running eight keys ahead.  The output is o/den times sigmoid(gate)
+// loads running kAhead keys ahead.  The output is o/den times sigmoid(gate)
 // (execution.rs:506-508).
 // ---------------------------------------------------------------------------
+template <int kAhead>
 __global__ __launch_bounds__(576) void k_q35_attn(Q35Rows Rw, const float *__restrict__ scores,
                                                   int ldsc, const float *__restrict__ z, int ldq,
                                                   const float *__restrict__ vc, size_t cache_seq,
@@ -991,38 +992,93 @@ __global__ __launch_bounds__(576) void k_q35_attn(Q35Rows Rw, const float *__res
   __syncthreads();
   if (tid == dthreads) {
     float den = 0.0f;
-    for (int t = 0; t < kv; t++) den = den * old[t] + sc[t];
+    int t = 0;
+    if constexpr (kAhead > 8) {
+      // whole groups of 8 keys, the next group's factors loading while the
+      // current one is folded in
+      float4 of[2], nf[2], on[2], nn[2];
+      auto get = [&](float4 (&o4)[2], float4 (&n4)[2], int g) {
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+          o4[u] = *reinterpret_cast<const float4 *>(old + 8 * g + 4 * u);
+          n4[u] = *reinterpret_cast<const float4 *>(sc + 8 * g + 4 * u);
+        }
+      };
+      const int full = kv / 8;
+      if (full) get(of, nf, 0);
+      for (int g = 0; g < full; g++) {
+        get(on, nn, min(g + 1, full - 1));
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+          den = den * of[u].x + nf[u].x;
+          den = den * of[u].y + nf[u].y;
+          den = den * of[u].z + nf[u].z;
+          den = den * of[u].w + nf[u].w;
+          of[u] = on[u];
+          nf[u] = nn[u];
+        }
+      }
+      t = full * 8;
+    }
+    for (; t < kv; t++) den = den * old[t] + sc[t];
     s_den = den;
   }
   float o = 0.0f;
   if (tid < D) {
-    // whole groups of 8 keys without branches, the next group's V values
-    // loading while the current group is folded in; then the tail
-    const float *vp = V + tid;
-    const int full = kv / 8;
-    float cur[8], nxt[8];
+    if constexpr (kAhead == 8) {
+      // whole groups of 8 keys without branches, the next group's V values
+      // loading while the current group is folded in; then the tail
+      const float *vp = V + tid;
+      const int full = kv / 8;
+      float cur[8], nxt[8];
 #pragma unroll
-    for (int j = 0; j < 8; j++) cur[j] = full ? vp[(size_t)j * kvw] : 0.0f;
-    for (int g = 0; g < full; g++) {
-      const int tn = min(g + 1, full - 1) * 8;
+      for (int j = 0; j < 8; j++) cur[j] = full ? vp[(size_t)j * kvw] : 0.0f;
+      for (int g = 0; g < full; g++) {
+        const int tn = min(g + 1, full - 1) * 8;
 #pragma unroll
-      for (int j = 0; j < 8; j++) nxt[j] = vp[(size_t)(tn + j) * kvw];
-      const float4 o0 = *reinterpret_cast<const float4 *>(old + 8 * g);
-      const float4 o1 = *reinterpret_cast<const float4 *>(old + 8 * g + 4);
-      const float4 n0 = *reinterpret_cast<const float4 *>(sc + 8 * g);
-      const float4 n1 = *reinterpret_cast<const float4 *>(sc + 8 * g + 4);
-      o = o * o0.x + n0.x * cur[0];
-      o = o * o0.y + n0.y * cur[1];
-      o = o * o0.z + n0.z * cur[2];
-      o = o * o0.w + n0.w * cur[3];
-      o = o * o1.x + n1.x * cur[4];
-      o = o * o1.y + n1.y * cur[5];
-      o = o * o1.z + n1.z * cur[6];
-      o = o * o1.w + n1.w * cur[7];
+        for (int j = 0; j < 8; j++) nxt[j] = vp[(size_t)(tn + j) * kvw];
+        const float4 o0 = *reinterpret_cast<const float4 *>(old + 8 * g);
+        const float4 o1 = *reinterpret_cast<const float4 *>(old + 8 * g + 4);
+        const float4 n0 = *reinterpret_cast<const float4 *>(sc + 8 * g);
+        const float4 n1 = *reinterpret_cast<const float4 *>(sc + 8 * g + 4);
+        o = o * o0.x + n0.x * cur[0];
+        o = o * o0.y + n0.y * cur[1];
+        o = o * o0.z + n0.z * cur[2];
+        o = o * o0.w + n0.w * cur[3];
+        o = o * o1.x + n1.x * cur[4];
+        o = o * o1.y + n1.y * cur[5];
+        o = o * o1.z + n1.z * cur[6];
+        o = o * o1.w + n1.w * cur[7];
 #pragma unroll
-      for (int j = 0; j < 8; j++) cur[j] = nxt[j];
+        for (int j = 0; j < 8; j++) cur[j] = nxt[j];
+      }
+      for (int t = full * 8; t < kv; t++) o = o * old[t] + sc[t] * vp[(size_t)t * kvw];
+    } else {
+      // groups of kAhead keys, the next group's V values loading while the
+      // current group is folded in; a last, partial group folds its own keys
+      const float *vp = V + tid;
+      const int groups = (kv + kAhead - 1) / kAhead;
+      float cur[kAhead], nxt[kAhead];
+#pragma unroll
+      for (int j = 0; j < kAhead; j++) cur[j] = vp[(size_t)min(j, kv - 1) * kvw];
+      for (int g = 0; g < groups; g++) {
+        const int t0 = g * kAhead;
+#pragma unroll
+        for (int j = 0; j < kAhead; j++) nxt[j] = vp[(size_t)min(t0 + kAhead + j, kv - 1) * kvw];
+#pragma unroll
+        for (int u = 0; u < kAhead; u += 4) {
+          if (t0 + u >= kv) break;
+          const float4 of = *reinterpret_cast<const float4 *>(old + t0 + u);
+          const float4 nf = *reinterpret_cast<const float4 *>(sc + t0 + u);
+          o = o * of.x + nf.x * cur[u];
+          if (t0 + u + 1 < kv) o = o * of.y + nf.y * cur[u + 1];
+          if (t0 + u + 2 < kv) o = o * of.z + nf.z * cur[u + 2];
+          if (t0 + u + 3 < kv) o = o * of.w + nf.w * cur[u + 3];
+        }
+#pragma unroll
+        for (int j = 0; j < kAhead; j++) cur[j] = nxt[j];
+      }
     }
-    for (int t = full * 8; t < kv; t++) o = o * old[t] + sc[t] * vp[(size_t)t * kvw];
   }
   __syncthreads();
   if (tid < D) {
@@ -1251,8 +1307,15 @@ void q35_attention(hipStream_t s, int rows, Q35Rows Rw, const float *q, const fl
   const int threads = ((D + kWave - 1) / kWave) * kWave + kWave;
   const int maxc4 = (max_context + 3) / 4 * 4;
   const size_t lds = (size_t)(3 * maxc4 + threads) * sizeof(float);
-  hipLaunchKernelGGL(k_q35_attn, dim3(rows, heads), dim3(threads), lds, s, Rw, scores, max_context,
-                     z, ldq, vc, cache_seq, heads, kv_heads, D, maxc4, out, ldo);
+  // few rows: the walk over the keys waits on memory, so 32 keys' V values are
+  // in flight per thread (16 decode rows over 32-448 keys: 35 -> 25 us); many rows
+  // hide that among themselves and keep the smaller form's occupancy
+  if (rows * heads <= 1024)
+    hipLaunchKernelGGL(k_q35_attn<32>, dim3(rows, heads), dim3(threads), lds, s, Rw, scores, max_context,
+                       z, ldq, vc, cache_seq, heads, kv_heads, D, maxc4, out, ldo);
+  else
+    hipLaunchKernelGGL(k_q35_attn<8>, dim3(rows, heads), dim3(threads), lds, s, Rw, scores, max_context,
+                       z, ldq, vc, cache_seq, heads, kv_heads, D, maxc4, out, ldo);
 }
 
 }  // namespace cohx
