@@ -41,6 +41,18 @@ inline size_t q35_tiled_index(size_t row, size_t k, size_t K) {
 
 enum Q35Epi { kQ35Store = 0, kQ35Residual = 1, kQ35Argmax = 2, kQ35Swiglu = 3 };
 
+// Up to kPieces device copies in one launch, passed by value.  Every source
+// and destination is 16-byte aligned.
+struct Q35Copy {
+  static constexpr int kPieces = 64;
+  struct Piece {
+    const float *src;
+    float *dst;
+    size_t floats;
+  } piece[kPieces];
+};
+void q35_copy(hipStream_t s, const Q35Copy &c, int pieces);
+
 void q35_embed(hipStream_t s, int rows, const uint16_t *embed, const uint32_t *tokens, int H,
                float *x);
 // out[r] = norm(x[src ? src[r] : r]) * (w + zc)

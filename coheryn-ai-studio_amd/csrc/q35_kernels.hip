@@ -1115,9 +1115,23 @@ __global__ __launch_bounds__(256) void k_q35_split(const float *__restrict__ x, 
       make_uint2(l[0] | (uint32_t)l[1] << 16, l[2] | (uint32_t)l[3] << 16);
 }
 
+// Copies of a snapshot (cohx_seq_fork): piece blockIdx.y, 16-byte words.
+__global__ __launch_bounds__(256) void k_q35_copy(Q35Copy c) {
+  const Q35Copy::Piece p = c.piece[blockIdx.y];
+  const u32x4q *src = reinterpret_cast<const u32x4q *>(p.src);
+  u32x4q *dst = reinterpret_cast<u32x4q *>(p.dst);
+  const size_t n = p.floats / 4, step = (size_t)gridDim.x * 256;
+  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += step) dst[i] = src[i];
+  for (size_t i = n * 4 + (size_t)blockIdx.x * 256 + threadIdx.x; i < p.floats; i += step) p.dst[i] = p.src[i];
+}
+
 }  // namespace
 
 // ---- launchers ---------------------------------------------------------------
+
+void q35_copy(hipStream_t s, const Q35Copy &c, int pieces) {
+  hipLaunchKernelGGL(k_q35_copy, dim3(64, pieces), dim3(256), 0, s, c);
+}
 
 void q35_embed(hipStream_t s, int rows, const uint16_t *embed, const uint32_t *tokens, int H,
                float *x) {
