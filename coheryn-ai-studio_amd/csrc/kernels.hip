@@ -14,8 +14,6 @@
 #include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
-#include <cstdio>
-#include <cstdlib>
 #include <type_traits>
 
 #include "device.h"
@@ -711,31 +709,45 @@ __global__ __launch_bounds__(64 * kW) void k_mv_q8s(MatrixView w, ActView act, i
 // last block the chains meet in LDS and sum + lanes[0] + ... + lanes[7] is
 // added in that order.  Q6_K has no min chain; its sum starts at +0 too.
 // ---------------------------------------------------------------------------
+// 16-bit pairs: bytes 1 and 3 of x, sign-extended (v_perm selectors 8 and 9
+// are the signs of bytes 1 and 3).
+typedef short s16x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ s16x2 odd_bytes(uint32_t x) {
+  return __builtin_bit_cast(s16x2, __builtin_amdgcn_perm(x, x, 0x09030801u));
+}
+// The eight products value * sub-group scale (|p| <= 4096, in 16 bits), split
+// as 128 hi + lo: values 0, 1 take scale byte 0, values 2, 3 byte 1, and so on,
+// so the pairs (0, 2) and (1, 3) of a word share one pair of scales.
 __device__ __forceinline__ void kq_split(uint2 q, uint32_t sc, long &hi, long &lo) {
-  uint32_t h[2] = {0u, 0u}, l[2] = {0u, 0u};
+  uint32_t h[2], l[2];
 #pragma unroll
-  for (int j = 0; j < 8; j++) {
-    const uint32_t word = j < 4 ? q.x : q.y;
-    const int v = (int)(int8_t)(word >> (8 * (j % 4)));
-    const int s = (int)(int8_t)(sc >> (8 * (j / 2)));
-    const int p = v * s;
-    h[j / 4] |= (uint32_t)((p >> 7) & 0xff) << (8 * (j % 4));
-    l[j / 4] |= (uint32_t)(p & 0x7f) << (8 * (j % 4));
+  for (int w = 0; w < 2; w++) {
+    const uint32_t x = w ? q.y : q.x;
+    const s16x2 s = odd_bytes(__builtin_amdgcn_perm(sc, sc, w ? 0x030c020cu : 0x010c000cu));
+    const s16x2 p02 = odd_bytes(x << 8) * s, p13 = odd_bytes(x) * s;
+    const uint32_t h02 = __builtin_bit_cast(uint32_t, (s16x2)(p02 >> 7)), h13 = __builtin_bit_cast(uint32_t, (s16x2)(p13 >> 7));
+    // bytes 0 and 2 of both pairs, in value order
+    h[w] = __builtin_amdgcn_perm(h13, h02, 0x06020400u);
+    l[w] = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, p13), __builtin_bit_cast(uint32_t, p02), 0x06020400u) &
+           0x7f7f7f7fu;
   }
   hi = (long)(((unsigned long)h[1] << 32) | h[0]);
   lo = (long)(((unsigned long)l[1] << 32) | l[0]);
 }
 
-template <int kEpi, int kNM>
+// The loads of a block run two blocks ahead of their use (each block used to
+// wait for its own: down at 32 rows 19.5 us, 11.4 now), and a workgroup takes
+// kNN batch tiles, which share each weight's scaling and split.
+template <int kEpi, int kNM, int kNN>
 __global__ __launch_bounds__(512) void k_mv_kq(MatrixView w, ActView act, int rows_b, int n_tiles,
                                                MatvecOut o) {
-  __shared__ float s_lane[8][kNM][256];
-  __shared__ float s_min[kNM][256];
-  __shared__ unsigned long long s_key[4][16];
+  __shared__ float s_lane[8][kNM * kNN][256];
+  __shared__ float s_min[kNM * kNN][256];
+  __shared__ unsigned long long s_key[kNN][4][16];
   const int lane = threadIdx.x % kWave, c = threadIdx.x / kWave;
-  const int units = w.mtiles / kNM;
-  const int group = blockIdx.x / (8 * n_tiles), rem = blockIdx.x % (8 * n_tiles);
-  const int nt = rem / 8, unit = group * 8 + rem % 8;
+  const int units = w.mtiles / kNM, groups = (n_tiles + kNN - 1) / kNN;
+  const int group = blockIdx.x / (8 * groups), rem = blockIdx.x % (8 * groups);
+  const int nt0 = rem / 8 * kNN, unit = group * 8 + rem % 8;
   if (unit >= units) return;
   const int nb = w.nb;
   const v4i zero = {0, 0, 0, 0};
@@ -744,119 +756,176 @@ __global__ __launch_bounds__(512) void k_mv_kq(MatrixView w, ActView act, int ro
   const int p = c * 32 + (lane % 32);
   const int mrow = 4 * ((p % 64) / 16) + p / 64, mcol = p % 16;
   const bool mown = w.has_min && lane < 32;
-  float L[kNM][4], S[kNM];
+  float L[kNM][kNN][4], S[kNM][kNN];
 #pragma unroll
-  for (int m = 0; m < kNM; m++) {
-    S[m] = 0.0f;
+  for (int m = 0; m < kNM; m++)
 #pragma unroll
-    for (int i = 0; i < 4; i++) L[m][i] = 0.0f;
-  }
-  for (int b = 0; b < nb; b++) {
-    const uint2 av = *reinterpret_cast<const uint2 *>(act.qs + kq_byte(nt, nb, b, c, lane, 0));
-    const long bop = (long)(((unsigned long)av.y << 32) | av.x);
-    const float da = act.kd[kq_row(nt, nb, b, lane % 16)];
+    for (int n = 0; n < kNN; n++) {
+      S[m][n] = 0.0f;
+#pragma unroll
+      for (int i = 0; i < 4; i++) L[m][n][i] = 0.0f;
+    }
+  struct Block {
+    uint2 av[kNN], qv[kNM], dw[kNM], mn[kNM];
+    float da[kNN], dam[kNN];
+    uint32_t sc[kNM];
+    u32x4v g[kNN][2];
+    uint16_t dm[kNM];
+  };
+  // batch tiles past the last repeat it, blocks past the last load it again
+  // (neither is used); the min chain's operands load in every lane
+  auto load = [&](Block &r, int b_) {
+    const int b = min(b_, nb - 1);
+#pragma unroll
+    for (int n = 0; n < kNN; n++) {
+      const int nt = min(nt0 + n, n_tiles - 1);
+      r.av[n] = *reinterpret_cast<const uint2 *>(act.qs + kq_byte(nt, nb, b, c, lane, 0));
+      r.da[n] = act.kd[kq_row(nt, nb, b, lane % 16)];
+    }
 #pragma unroll
     for (int m = 0; m < kNM; m++) {
       const size_t tile = (size_t)unit * kNM + m;
-      const uint2 qv = *reinterpret_cast<const uint2 *>(w.qs + kq_byte(tile, nb, b, c, lane, 0));
-      const uint32_t sc = w.ksc[kq_row(tile, nb, b, 0) * 4 + lane];
-      const uint2 dw4 = *reinterpret_cast<const uint2 *>(w.ds + kq_row(tile, nb, b, 4 * (lane / 16)));
-      long hi, lo;
-      kq_split(qv, sc, hi, lo);
-      v4i ih = __builtin_amdgcn_mfma_i32_16x16x32_i8(hi, bop, zero, 0, 0, 0);
-#pragma unroll
-      for (int i = 0; i < 4; i++) ih[i] *= 128;
-      const v4i is = __builtin_amdgcn_mfma_i32_16x16x32_i8(lo, bop, ih, 0, 0, 0);
-      const uint16_t dws[4] = {(uint16_t)dw4.x, (uint16_t)(dw4.x >> 16), (uint16_t)dw4.y,
-                               (uint16_t)(dw4.y >> 16)};
-#pragma unroll
-      for (int i = 0; i < 4; i++) L[m][i] = fmaf(h2f(dws[i]) * da, (float)is[i], L[m][i]);
+      r.qv[m] = *reinterpret_cast<const uint2 *>(w.qs + kq_byte(tile, nb, b, c, lane, 0));
+      r.sc[m] = w.ksc[kq_row(tile, nb, b, 0) * 4 + lane];
+      r.dw[m] = *reinterpret_cast<const uint2 *>(w.ds + kq_row(tile, nb, b, 4 * (lane / 16)));
     }
-    if (mown) {
-      const size_t ar = kq_row(nt, nb, b, mcol);
-      const float dam = act.kd[ar];
-      const uint4 g0 = *reinterpret_cast<const uint4 *>(act.ksum + ar * 16);
-      const uint4 g1 = *reinterpret_cast<const uint4 *>(act.ksum + ar * 16 + 8);
-      const uint32_t gw[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
+    if (w.has_min) {
+#pragma unroll
+      for (int n = 0; n < kNN; n++) {
+        const size_t ar = kq_row(min(nt0 + n, n_tiles - 1), nb, b, mcol);
+        r.dam[n] = act.kd[ar];
+        r.g[n][0] = *reinterpret_cast<const u32x4v *>(act.ksum + ar * 16);
+        r.g[n][1] = *reinterpret_cast<const u32x4v *>(act.ksum + ar * 16 + 8);
+      }
 #pragma unroll
       for (int m = 0; m < kNM; m++) {
         const size_t wr = kq_row((size_t)unit * kNM + m, nb, b, mrow);
-        const uint2 mn = *reinterpret_cast<const uint2 *>(w.kmin + wr * 8);
-        int ms = 0;
-#pragma unroll
-        for (int g = 0; g < 8; g++) {
-          const int mg = (int)(((g < 4 ? mn.x : mn.y) >> (8 * (g % 4))) & 0xffu);
-          const int gsum = (int)(int16_t)(gw[g] & 0xffffu) + (int)(int16_t)(gw[g] >> 16);
-          ms += mg * gsum;
-        }
-        S[m] = fmaf(-(h2f(w.kdm[wr]) * dam), (float)ms, S[m]);
+        r.mn[m] = *reinterpret_cast<const uint2 *>(w.kmin + wr * 8);
+        r.dm[m] = w.kdm[wr];
       }
+    }
+  };
+  auto use = [&](const Block &r) {
+    long hi[kNM], lo[kNM];
+#pragma unroll
+    for (int m = 0; m < kNM; m++) kq_split(r.qv[m], r.sc[m], hi[m], lo[m]);
+#pragma unroll
+    for (int n = 0; n < kNN; n++) {
+      const long bop = (long)(((unsigned long)r.av[n].y << 32) | r.av[n].x);
+#pragma unroll
+      for (int m = 0; m < kNM; m++) {
+        v4i ih = __builtin_amdgcn_mfma_i32_16x16x32_i8(hi[m], bop, zero, 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 4; i++) ih[i] *= 128;
+        const v4i is = __builtin_amdgcn_mfma_i32_16x16x32_i8(lo[m], bop, ih, 0, 0, 0);
+        const uint16_t dws[4] = {(uint16_t)r.dw[m].x, (uint16_t)(r.dw[m].x >> 16), (uint16_t)r.dw[m].y,
+                                 (uint16_t)(r.dw[m].y >> 16)};
+#pragma unroll
+        for (int i = 0; i < 4; i++) L[m][n][i] = fmaf(h2f(dws[i]) * r.da[n], (float)is[i], L[m][n][i]);
+      }
+    }
+    if (mown) {
+      // sum_g min_g * (s_2g + s_2g+1): one 16-bit pair dot product a group
+#pragma unroll
+      for (int m = 0; m < kNM; m++) {
+        s16x2 mg[8];
+#pragma unroll
+        for (int g = 0; g < 8; g++) {  // min_g (0..63) in both halves
+          const uint32_t x = g < 4 ? r.mn[m].x : r.mn[m].y, i = g % 4;
+          mg[g] = __builtin_bit_cast(s16x2, __builtin_amdgcn_perm(x, x, 0x0c000c00u | i << 16 | i));
+        }
+#pragma unroll
+        for (int n = 0; n < kNN; n++) {
+          int ms = 0;
+#pragma unroll
+          for (int g = 0; g < 8; g++) {
+            const uint32_t pair = r.g[n][g / 4][g % 4];
+            ms = __builtin_amdgcn_sdot2(__builtin_bit_cast(s16x2, pair), mg[g], ms, false);
+          }
+          S[m][n] = fmaf(-(h2f(r.dm[m]) * r.dam[n]), (float)ms, S[m][n]);
+        }
+      }
+    }
+  };
+  constexpr int kD = 3;
+  Block ring[kD];
+#pragma unroll
+  for (int i = 0; i < kD - 1; i++) load(ring[i], i);
+  for (int b0 = 0; b0 < nb; b0 += kD) {
+#pragma unroll
+    for (int u = 0; u < kD; u++) {
+      load(ring[(u + kD - 1) % kD], b0 + u + kD - 1);
+      if (b0 + u < nb) use(ring[u]);
     }
   }
 #pragma unroll
-  for (int m = 0; m < kNM; m++) {
+  for (int m = 0; m < kNM; m++)
 #pragma unroll
-    for (int i = 0; i < 4; i++) s_lane[c][m][i * 64 + lane] = L[m][i];
-    if (lane < 32) s_min[m][p] = S[m];
-  }
+    for (int n = 0; n < kNN; n++) {
+#pragma unroll
+      for (int i = 0; i < 4; i++) s_lane[c][m * kNN + n][i * 64 + lane] = L[m][n][i];
+      if (lane < 32) s_min[m * kNN + n][p] = S[m][n];
+    }
   __syncthreads();
-  // ---- the chains meet; then the epilogue (as k_mv_q8s)
-  const int t = threadIdx.x, prow = 4 * ((t % 64) / 16) + t / 64, pcol = t % 16;
-  float acc[kNM];
+  // ---- the chains meet; then the epilogue (as k_mv_q8s): threads 0..255 take
+  // batch tile nt0, 256..511 nt0 + 1, ...
+  for (int n = threadIdx.x / 256; n < kNN; n += 2) {
+    const int t = threadIdx.x % 256, prow = 4 * ((t % 64) / 16) + t / 64, pcol = t % 16;
+    float acc[kNM];
 #pragma unroll
-  for (int m = 0; m < kNM; m++) {
-    acc[m] = 0.0f;
-    if (t < 256) {
-      float v = s_min[m][t];
+    for (int m = 0; m < kNM; m++) {
+      float v = s_min[m * kNN + n][t];
 #pragma unroll
-      for (int cc = 0; cc < 8; cc++) v = v + s_lane[cc][m][t];
+      for (int cc = 0; cc < 8; cc++) v = v + s_lane[cc][m * kNN + n][t];
       acc[m] = v;
     }
-  }
-  const int r = nt * 16 + pcol;
-  const bool rvalid = t < 256 && r < rows_b;
-  const int er = (rvalid && o.err_rows) ? (int)o.err_rows[r] : r;
-  bool bad = false;
-  if constexpr (kEpi == kEpiArgmax) {
-    const int row = unit * 16 + prow;
-    const bool valid = rvalid && row < w.rows;
-    const float v = acc[0];
-    if (valid) {
-      bad = !finitef(v);
-      if (o.logits) o.logits[(size_t)r * w.rows + row] = v;
-    }
-    unsigned long long key = valid ? argmax_key(v, row) : 0ull;
-    unsigned long long x = __shfl_xor(key, 16, kWave);
-    key = x > key ? x : key;
-    x = __shfl_xor(key, 32, kWave);
-    key = x > key ? x : key;
-    if (t < 256 && lane < 16) s_key[c][lane] = key;
-    __syncthreads();
-    if (t < 16) {
-      unsigned long long best = s_key[0][t];
-#pragma unroll
-      for (int i = 1; i < 4; i++) best = s_key[i][t] > best ? s_key[i][t] : best;
-      if (nt * 16 + t < rows_b) o.argmax[(size_t)(nt * 16 + t) * units + unit] = best;
-    }
-  } else if (rvalid) {
-    const int row = unit * 16 + prow;
-    if (kEpi == kEpiSwiglu) {
-      if (row < w.rows / 2) {
-        const float g = acc[0], u = acc[kNM - 1];
-        bad = !finitef(g) || !finitef(u);
-        o.out[(size_t)r * o.ld + row] = (g / (1.0f + exp_f32(-g))) * u;
-      }
-    } else if (row < w.rows) {
+    const int r = (nt0 + n) * 16 + pcol, row = unit * 16 + prow;
+    const bool rvalid = r < rows_b;
+    const int er = (rvalid && o.err_rows) ? (int)o.err_rows[r] : r;
+    bool bad = false;
+    if constexpr (kEpi == kEpiArgmax) {
+      const bool valid = rvalid && row < w.rows;
       const float v = acc[0];
-      bad = !finitef(v);
-      float *q = o.out + (size_t)r * o.ld + row;
-      if (kEpi == kEpiResidual)
-        *q = *q + v;
-      else
-        *q = v;
+      if (valid) {
+        bad = !finitef(v);
+        if (o.logits) o.logits[(size_t)r * w.rows + row] = v;
+      }
+      unsigned long long key = valid ? argmax_key(v, row) : 0ull;
+      unsigned long long x = __shfl_xor(key, 16, kWave);
+      key = x > key ? x : key;
+      x = __shfl_xor(key, 32, kWave);
+      key = x > key ? x : key;
+      if (lane < 16) s_key[n][t / kWave][lane] = key;
+    } else if (rvalid) {
+      if (kEpi == kEpiSwiglu) {
+        if (row < w.rows / 2) {
+          const float g = acc[0], u = acc[kNM - 1];
+          bad = !finitef(g) || !finitef(u);
+          o.out[(size_t)r * o.ld + row] = (g / (1.0f + exp_f32(-g))) * u;
+        }
+      } else if (row < w.rows) {
+        const float v = acc[0];
+        bad = !finitef(v);
+        float *q = o.out + (size_t)r * o.ld + row;
+        if (kEpi == kEpiResidual)
+          *q = *q + v;
+        else
+          *q = v;
+      }
+    }
+    if (bad) atomicOr(&o.row_err[er], kErrNonFinite);
+  }
+  if constexpr (kEpi == kEpiArgmax) {
+    __syncthreads();
+    if (threadIdx.x < 16 * kNN) {
+      const int n = threadIdx.x / 16, t = threadIdx.x % 16;
+      unsigned long long best = s_key[n][0][t];
+#pragma unroll
+      for (int i = 1; i < 4; i++) best = s_key[n][i][t] > best ? s_key[n][i][t] : best;
+      const int r = (nt0 + n) * 16 + t;
+      if (r < rows_b) o.argmax[(size_t)r * units + unit] = best;
     }
   }
-  if (bad) atomicOr(&o.row_err[er], kErrNonFinite);
 }
 
 // ---------------------------------------------------------------------------
@@ -3162,8 +3231,20 @@ bool launch_matvec_swiglu_f16(hipStream_t s, const MatrixView &w, const ActView 
 template <int kEpi, int kNM>
 static void mv_kq(hipStream_t s, const MatrixView &w, const ActView &act, int rows_b, const MatvecOut &o) {
   const int units = w.mtiles / kNM, n_tiles = (rows_b + 15) / 16;
-  launch_k((k_mv_kq<kEpi, kNM>), dim3((units + 7) / 8 * 8 * n_tiles), dim3(512), 0, s, w, act, rows_b,
-           n_tiles, o);
+  auto go = [&](auto nn) {
+    constexpr int kNN = decltype(nn)::value;
+    const int groups = (n_tiles + kNN - 1) / kNN;
+    launch_k((k_mv_kq<kEpi, kNM, kNN>), dim3((units + 7) / 8 * 8 * groups), dim3(512), 0, s, w, act, rows_b, n_tiles,
+             o);
+  };
+  // one batch tile per workgroup keeps the grid wide at few rows (down at 32
+  // rows: 11.4 us, 16.1 as two, 19.9 as three); from eight tiles on the shared
+  // loads and splits win (387 rows: 50.9 as one, 41.9 as two, 37.4 as three;
+  // three tiles of a gate and up pair would leave one wave a SIMD)
+  if (n_tiles >= 8)
+    go(std::integral_constant<int, kNM == 2 ? 2 : 3>{});
+  else
+    go(std::integral_constant<int, 1>{});
 }
 
 bool launch_matvec(hipStream_t s, Epilogue epi, const MatrixView &w, const ActView &act,
