@@ -1338,11 +1338,13 @@ __global__ __launch_bounds__(512 * kU) void k_mv_q8w(MatrixView w, ActView act, 
 // block scales are copied to LDS once per workgroup, in the same memory round
 // trip.  Workgroups of one block q sit on one XCD (blockIdx % 8), so the
 // weight tiles shared by its batch groups are fetched into that L2 once.
+// hout (a down projection with another operand form): the f32 SwiGLU rows
+// [rows_b][F] instead of the Q8_0 operand.
 // ---------------------------------------------------------------------------
 template <int kFmt, int kNB, int kNN, int kMaxPairs, bool kExact = false>
 __global__ __launch_bounds__(256 * kNB) void k_mv_gu(MatrixView w, ActView act, int rows_b, int n_tiles,
                                                      uint32_t *row_err, const uint32_t *err_rows,
-                                                     ActView qout, int qout_nbp) {
+                                                     ActView qout, int qout_nbp, float *hout) {
   constexpr int kBT = kNB * kNN;  // batch tiles per workgroup
   extern __shared__ uint4 smem[];
   __shared__ uint64_t s_tab[32];
@@ -1474,7 +1476,15 @@ __global__ __launch_bounds__(256 * kNB) void k_mv_gu(MatrixView w, ActView act, 
       bad |= rvalid && (!finitef(g) || !finitef(up));
       v[e] = (g / (1.0f + exp_f32_tab(-g, s_tab))) * up;
     }
-    bad |= quant_group_q8<16>(v, rvalid, r, q * 4 + k, qout_nbp, qout);
+    if (hout) {
+      if (rvalid) {
+        float4 *dst = reinterpret_cast<float4 *>(hout + (size_t)r * (w.rows / 2) + q * 32 + 8 * k);
+        dst[0] = make_float4(v[0], v[1], v[2], v[3]);
+        dst[1] = make_float4(v[4], v[5], v[6], v[7]);
+      }
+    } else {
+      bad |= quant_group_q8<16>(v, rvalid, r, q * 4 + k, qout_nbp, qout);
+    }
     if (bad) atomicOr(&row_err[err_rows ? (int)err_rows[r] : r], kErrNonFinite);
   }
 }
@@ -2927,13 +2937,37 @@ void launch_quant_act(hipStream_t s, int rows, const float *src, int K, int act_
     launch_k(k_quant_act<1>, dim3(rows, splits), dim3(256), 0, s, src, K, nbp, act, row_err);
 }
 
+// k_mv_gu at fewer than eight batch tiles: one wave per (weight tile, batch
+// tile), every CU busy.  K = 896 (Qwen2.5-0.5B's hidden size) gets a kernel
+// built for exactly its 14 block pairs (straight-line block loops).
+static void mv_gu(hipStream_t s, const MatrixView &w, const ActView &act, int rows_b, const MatvecOut &o,
+                  const ActView &qout, int qout_nbp, float *hout) {
+  constexpr int kWPairs = 16, kExactPairs = 14;
+  const int n_tiles = (rows_b + 15) / 16, nq = w.mtiles / 4, npairs = w.nbp / 2;
+  const size_t items = (size_t)npairs * 64 + 4 * (size_t)w.nbp * 2 + (size_t)w.nbp * 2;
+  const size_t lds = items * 16 > 4096 ? items * 16 : 4096;
+  const dim3 grid((nq + 7) / 8 * 8 * n_tiles);
+  if (w.dtype == 8 && npairs == kExactPairs)
+    launch_k((k_mv_gu<8, 1, 1, kExactPairs, true>), grid, dim3(256), lds, s, w, act, rows_b, n_tiles, o.row_err,
+             o.err_rows, qout, qout_nbp, hout);
+  else if (w.dtype == 8)
+    launch_k((k_mv_gu<8, 1, 1, kWPairs>), grid, dim3(256), lds, s, w, act, rows_b, n_tiles, o.row_err, o.err_rows,
+             qout, qout_nbp, hout);
+  else
+    launch_k((k_mv_gu<2, 1, 1, kWPairs>), grid, dim3(256), lds, s, w, act, rows_b, n_tiles, o.row_err, o.err_rows,
+             qout, qout_nbp, hout);
+}
+
 template <int kEpi, int kNM, int kFmt>
 static bool mv_q8(hipStream_t s, const MatrixView &w, const ActView &act, int rows_b,
                   const MatvecOut &o) {
   const int units = w.mtiles / kNM;
   const int n_tiles = (rows_b + 15) / 16;
   constexpr int kWPairs = 16;  // k_mv_q8w: K <= 1024
-  if (kEpi == kEpiSwiglu && w.nbp <= 2 * kWPairs) {
+  if (kEpi == kEpiSwiglu && w.nbp <= 2 * kWPairs && n_tiles < 8 && w.rows / 2 % 64 == 0 && o.ld == w.rows / 2) {
+    // (32 rows, Q5_0 gate+up before a Q4_K down projection: 15.0 -> 10.0 us)
+    mv_gu(s, w, act, rows_b, o, ActView{}, 0, o.out);
+  } else if (kEpi == kEpiSwiglu && w.nbp <= 2 * kWPairs) {
     // gate+up at short K: the unit's weights in LDS, B operands in registers
     const int by = (n_tiles + 7) / 8;
     const int nthreads = 64 * (n_tiles < 8 ? n_tiles : 8);
@@ -3307,20 +3341,7 @@ bool launch_matvec_swiglu_q8(hipStream_t s, const MatrixView &w, const ActView &
   // the epilogue writes whole block pairs of the down projection's operand
   if (qout_nbp != ((F / 32 + 1) & ~1)) return false;
   if (n_tiles < 8) {
-    // few batch tiles: one wave per (weight tile, batch tile), every CU busy
-    const int nq = w.mtiles / 4, npairs = w.nbp / 2;
-    const size_t items = (size_t)npairs * 64 + 4 * (size_t)w.nbp * 2 + (size_t)w.nbp * 2;
-    const size_t lds = items * 16 > 4096 ? items * 16 : 4096;
-    const dim3 grid((nq + 7) / 8 * 8 * n_tiles);
-    if (w.dtype == 8 && npairs == kExactPairs)
-      launch_k((k_mv_gu<8, 1, 1, kExactPairs, true>), grid, dim3(256), lds, s, w, act, rows_b, n_tiles, o.row_err,
-               o.err_rows, qout, qout_nbp);
-    else if (w.dtype == 8)
-      launch_k((k_mv_gu<8, 1, 1, kWPairs>), grid, dim3(256), lds, s, w, act, rows_b, n_tiles, o.row_err, o.err_rows,
-               qout, qout_nbp);
-    else
-      launch_k((k_mv_gu<2, 1, 1, kWPairs>), grid, dim3(256), lds, s, w, act, rows_b, n_tiles, o.row_err, o.err_rows,
-               qout, qout_nbp);
+    mv_gu(s, w, act, rows_b, o, qout, qout_nbp, nullptr);
     return true;
   }
   // eight batch tiles and more: the unit pair's weights shared through LDS
