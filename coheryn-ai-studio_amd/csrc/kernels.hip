@@ -2750,15 +2750,18 @@ __global__ __launch_bounds__(64 * kG) void k_attn_chunk(StepDims d, const int4 *
 // Pass 4: chunks combined in order, rounded to f32, and prepared as the
 // operand of attn_output (each head's D elements hold whole Q8_0 blocks).
 template <int kAct>
-__global__ __launch_bounds__(128) void k_attn_combine(StepDims d,
+__global__ __launch_bounds__(256) void k_attn_combine(StepDims d,
                                                       const uint32_t *__restrict__ row_pos,
                                                       const double *__restrict__ partial, int nbp,
                                                       ActView act, uint32_t *row_err) {
-  __shared__ float o_s[128];
-  const int r = blockIdx.x, h = blockIdx.y, j = threadIdx.x;
+  __shared__ float s_o[256];
+  const int tph = (d.D + kWave - 1) / kWave * kWave;  // threads per head
+  const int r = blockIdx.x, j = threadIdx.x % tph;
+  const int h = blockIdx.y * ((int)blockDim.x / tph) + threadIdx.x / tph;
+  float *o_s = s_o + threadIdx.x / tph * tph;
   const int kv = (int)row_pos[r] + 1, nch = (kv + kChunk - 1) / kChunk;
   const double *pp = partial + ((size_t)r * d.NH + h) * d.max_chunks * d.D;
-  const bool active = j < d.D;
+  const bool live = h < d.NH, active = live && j < d.D;
   double acc = 0.0;
   const bool direct = d.row_skip && d.row_skip[r];
   if (active && !direct) {
@@ -2820,7 +2823,7 @@ __global__ __launch_bounds__(128) void k_attn_combine(StepDims d,
     float v[8];
 #pragma unroll
     for (int i = 0; i < 8; i++) v[i] = j < ng ? o_s[j * 8 + i] : 0.0f;
-    if (j < ((ng + 3) & ~3))
+    if (live && j < ((ng + 3) & ~3))
       bad |= quant_group_q8<1, kAct == kActQ8H>(v, j < ng, r, h * ng + j, nbp, act);
   } else if (kAct == kActF32) {  // f32 rows for a following Q8_K quantizer
     if (active) act.f32[(size_t)r * d.H + h * d.D + j] = o;
@@ -3488,19 +3491,20 @@ void launch_attn_chunk(hipStream_t s, int n_tiles, const StepDims &d, const int4
 void launch_attn_combine(hipStream_t s, int rows, const StepDims &d, const uint32_t *row_pos,
                          const double *partial, int act_dtype, int nbp, ActView act,
                          uint32_t *row_err) {
-  const int threads = ((d.D + kWave - 1) / kWave) * kWave;
+  // a workgroup of one head, or of 256 threads' heads where (row, head)
+  // workgroups number in the ten thousands and their dispatch sets the pace
+  // (2,616 rows x 14 heads: 19.4 -> 17.0 us)
+  const int tph = ((d.D + kWave - 1) / kWave) * kWave;
+  const int heads = rows * d.NH >= 8192 ? 256 / tph : 1;
+  const dim3 grid(rows, (d.NH + heads - 1) / heads), block(heads * tph);
   if (act_dtype == kActQ8)
-    launch_k(k_attn_combine<kActQ8>, dim3(rows, d.NH), dim3(threads), 0, s, d, row_pos,
-                       partial, nbp, act, row_err);
+    launch_k(k_attn_combine<kActQ8>, grid, block, 0, s, d, row_pos, partial, nbp, act, row_err);
   else if (act_dtype == kActQ8H)
-    launch_k(k_attn_combine<kActQ8H>, dim3(rows, d.NH), dim3(threads), 0, s, d, row_pos,
-                       partial, nbp, act, row_err);
+    launch_k(k_attn_combine<kActQ8H>, grid, block, 0, s, d, row_pos, partial, nbp, act, row_err);
   else if (act_dtype == kActF32)
-    launch_k(k_attn_combine<kActF32>, dim3(rows, d.NH), dim3(threads), 0, s, d, row_pos,
-                       partial, nbp, act, row_err);
+    launch_k(k_attn_combine<kActF32>, grid, block, 0, s, d, row_pos, partial, nbp, act, row_err);
   else
-    launch_k(k_attn_combine<1>, dim3(rows, d.NH), dim3(threads), 0, s, d, row_pos,
-                       partial, nbp, act, row_err);
+    launch_k(k_attn_combine<1>, grid, block, 0, s, d, row_pos, partial, nbp, act, row_err);
 }
 
 void launch_fill_synthetic(hipStream_t s, float *kpool, float *vpool, size_t layer_stride,
