@@ -1338,10 +1338,10 @@ __global__ __launch_bounds__(512 * kU) void k_mv_q8w(MatrixView w, ActView act, 
 // block scales are copied to LDS once per workgroup, in the same memory round
 // trip.  Workgroups of one block q sit on one XCD (blockIdx % 8), so the
 // weight tiles shared by its batch groups are fetched into that L2 once.
-// hout (a down projection with another operand form): the f32 SwiGLU rows
-// [rows_b][F] instead of the Q8_0 operand.
+// kRows (a down projection with another operand form): the f32 SwiGLU rows
+// [rows_b][F] go to hout instead of the Q8_0 operand.
 // ---------------------------------------------------------------------------
-template <int kFmt, int kNB, int kNN, int kMaxPairs, bool kExact = false>
+template <int kFmt, int kNB, int kNN, int kMaxPairs, bool kExact, bool kRows>
 __global__ __launch_bounds__(256 * kNB) void k_mv_gu(MatrixView w, ActView act, int rows_b, int n_tiles,
                                                      uint32_t *row_err, const uint32_t *err_rows,
                                                      ActView qout, int qout_nbp, float *hout) {
@@ -1476,7 +1476,7 @@ __global__ __launch_bounds__(256 * kNB) void k_mv_gu(MatrixView w, ActView act, 
       bad |= rvalid && (!finitef(g) || !finitef(up));
       v[e] = (g / (1.0f + exp_f32_tab(-g, s_tab))) * up;
     }
-    if (hout) {
+    if constexpr (kRows) {
       if (rvalid) {
         float4 *dst = reinterpret_cast<float4 *>(hout + (size_t)r * (w.rows / 2) + q * 32 + 8 * k);
         dst[0] = make_float4(v[0], v[1], v[2], v[3]);
@@ -2749,19 +2749,21 @@ __global__ __launch_bounds__(64 * kG) void k_attn_chunk(StepDims d, const int4 *
 
 // Pass 4: chunks combined in order, rounded to f32, and prepared as the
 // operand of attn_output (each head's D elements hold whole Q8_0 blocks).
-template <int kAct>
-__global__ __launch_bounds__(256) void k_attn_combine(StepDims d,
-                                                      const uint32_t *__restrict__ row_pos,
-                                                      const double *__restrict__ partial, int nbp,
-                                                      ActView act, uint32_t *row_err) {
-  __shared__ float s_o[256];
-  const int tph = (d.D + kWave - 1) / kWave * kWave;  // threads per head
-  const int r = blockIdx.x, j = threadIdx.x % tph;
-  const int h = blockIdx.y * ((int)blockDim.x / tph) + threadIdx.x / tph;
-  float *o_s = s_o + threadIdx.x / tph * tph;
+// kWide: blockDim.y heads per workgroup, each on whole waves; else one head,
+// with nothing ahead of the first load that depends on the block's shape
+// (heads taken from the thread id by division cost decode steps about 0.5%).
+template <int kAct, bool kWide>
+__global__ __launch_bounds__(kWide ? 256 : 128) void k_attn_combine(StepDims d,
+                                                                    const uint32_t *__restrict__ row_pos,
+                                                                    const double *__restrict__ partial, int nbp,
+                                                                    ActView act, uint32_t *row_err) {
+  __shared__ float s_o[kWide ? 256 : 128];
+  const int sub = kWide ? __builtin_amdgcn_readfirstlane(threadIdx.y) : 0;
+  const int r = blockIdx.x, j = threadIdx.x, h = kWide ? blockIdx.y * blockDim.y + sub : blockIdx.y;
+  float *o_s = s_o + (kWide ? sub * blockDim.x : 0);
   const int kv = (int)row_pos[r] + 1, nch = (kv + kChunk - 1) / kChunk;
   const double *pp = partial + ((size_t)r * d.NH + h) * d.max_chunks * d.D;
-  const bool live = h < d.NH, active = live && j < d.D;
+  const bool live = !kWide || h < d.NH, active = live && j < d.D;
   double acc = 0.0;
   const bool direct = d.row_skip && d.row_skip[r];
   if (active && !direct) {
@@ -2950,15 +2952,24 @@ static void mv_gu(hipStream_t s, const MatrixView &w, const ActView &act, int ro
   const size_t items = (size_t)npairs * 64 + 4 * (size_t)w.nbp * 2 + (size_t)w.nbp * 2;
   const size_t lds = items * 16 > 4096 ? items * 16 : 4096;
   const dim3 grid((nq + 7) / 8 * 8 * n_tiles);
-  if (w.dtype == 8 && npairs == kExactPairs)
-    launch_k((k_mv_gu<8, 1, 1, kExactPairs, true>), grid, dim3(256), lds, s, w, act, rows_b, n_tiles, o.row_err,
-             o.err_rows, qout, qout_nbp, hout);
-  else if (w.dtype == 8)
-    launch_k((k_mv_gu<8, 1, 1, kWPairs>), grid, dim3(256), lds, s, w, act, rows_b, n_tiles, o.row_err, o.err_rows,
-             qout, qout_nbp, hout);
+  // a compile-time choice: as a branch on hout the epilogue cost the Q8_0 form
+  // about 0.5% of a decode step
+  auto go = [&](auto rows) {
+    constexpr bool kRows = decltype(rows)::value;
+    if (w.dtype == 8 && npairs == kExactPairs)
+      launch_k((k_mv_gu<8, 1, 1, kExactPairs, true, kRows>), grid, dim3(256), lds, s, w, act, rows_b, n_tiles,
+               o.row_err, o.err_rows, qout, qout_nbp, hout);
+    else if (w.dtype == 8)
+      launch_k((k_mv_gu<8, 1, 1, kWPairs, false, kRows>), grid, dim3(256), lds, s, w, act, rows_b, n_tiles,
+               o.row_err, o.err_rows, qout, qout_nbp, hout);
+    else
+      launch_k((k_mv_gu<2, 1, 1, kWPairs, false, kRows>), grid, dim3(256), lds, s, w, act, rows_b, n_tiles,
+               o.row_err, o.err_rows, qout, qout_nbp, hout);
+  };
+  if (hout)
+    go(std::true_type());
   else
-    launch_k((k_mv_gu<2, 1, 1, kWPairs>), grid, dim3(256), lds, s, w, act, rows_b, n_tiles, o.row_err, o.err_rows,
-             qout, qout_nbp, hout);
+    go(std::false_type());
 }
 
 template <int kEpi, int kNM, int kFmt>
@@ -3495,16 +3506,24 @@ void launch_attn_combine(hipStream_t s, int rows, const StepDims &d, const uint3
   // workgroups number in the ten thousands and their dispatch sets the pace
   // (2,616 rows x 14 heads: 19.4 -> 17.0 us)
   const int tph = ((d.D + kWave - 1) / kWave) * kWave;
-  const int heads = rows * d.NH >= 8192 ? 256 / tph : 1;
-  const dim3 grid(rows, (d.NH + heads - 1) / heads), block(heads * tph);
+  const bool wide = rows * d.NH >= 8192;
+  const int heads = wide ? 256 / tph : 1;
+  const dim3 grid(rows, (d.NH + heads - 1) / heads), block(tph, heads);
+  auto go = [&](auto kact) {
+    constexpr int kAct = decltype(kact)::value;
+    if (wide)
+      launch_k((k_attn_combine<kAct, true>), grid, block, 0, s, d, row_pos, partial, nbp, act, row_err);
+    else
+      launch_k((k_attn_combine<kAct, false>), grid, block, 0, s, d, row_pos, partial, nbp, act, row_err);
+  };
   if (act_dtype == kActQ8)
-    launch_k(k_attn_combine<kActQ8>, grid, block, 0, s, d, row_pos, partial, nbp, act, row_err);
+    go(std::integral_constant<int, kActQ8>());
   else if (act_dtype == kActQ8H)
-    launch_k(k_attn_combine<kActQ8H>, grid, block, 0, s, d, row_pos, partial, nbp, act, row_err);
+    go(std::integral_constant<int, kActQ8H>());
   else if (act_dtype == kActF32)
-    launch_k(k_attn_combine<kActF32>, grid, block, 0, s, d, row_pos, partial, nbp, act, row_err);
+    go(std::integral_constant<int, kActF32>());
   else
-    launch_k(k_attn_combine<1>, grid, block, 0, s, d, row_pos, partial, nbp, act, row_err);
+    go(std::integral_constant<int, 1>());
 }
 
 void launch_fill_synthetic(hipStream_t s, float *kpool, float *vpool, size_t layer_stride,
