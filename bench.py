@@ -580,10 +580,10 @@ def summarize_c5_trace(trace_csv, bench_json, mfma_csv=None):
         print(f"| {name} | {gx} | {len(d)} | {sum(d) / len(d):.2f} | {min(d):.2f} | {max(d):.2f} | "
               f"{sum(d) / 1e3:.2f} |")
     print("\nThe 30 largest (kernel, grid) groups by total time, over the three runs.  Grid y of the\n"
-          "matvec kernels counts row groups: `k_q35_mvpc` 36864x4 and `k_q35_mvd` 131584x1 / 114688x1\n"
-          "are the 16-row steps of the one-token schedule (o/out/down projections; mix; gate+up with SwiGLU, `k_q35_mvd<3, ...>`),\n"
-          "`k_q35_mvd<2, ...>` is the LM head with its argmax, and `k_q35_mv` with grid y in the hundreds\n"
-          "are the 256-token prompt chunks (up to 4096 rows) of the exact run; `k_gemm<1, true, ...>` is\n"
+          "matvec kernels counts groups of 4, 8 or 16 rows: `k_q35_mv<1, ...>` is the o/out/down projections,\n"
+          "`k_q35_mv<0, ...>` mix, `k_q35_mv<3, ...>` gate+up with SwiGLU, `k_q35_mv<2, ...>` the LM head with\n"
+          "its argmax; those with grid y in the hundreds are the 256-token prompt chunks (up to 4096 rows) of\n"
+          "the exact run; `k_gemm<1, true, ...>` is\n"
           "the regime's matrix-core GEMM over hi/lo operands, `k_q35_split` their split.\n\n"
           f"Summary: `python bench.py --summarize-c5-trace <dir>/<name>_kernel_trace.csv <bench stdout> "
           f"[<mfma counter_collection.csv>]`")
