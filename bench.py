@@ -868,7 +868,7 @@ def run_c5(seed, cpu_steps, threads, with_cpu=True):
         "bound": "hbm", "bytes_per_step": sb, "achieved": sb / es_s / 1e9, "peak": HBM_PEAK / 1e9,
         "unit": "GB/s", "frac": sb / es_s / HBM_PEAK,
         "note": "weights once plus each sequence's delta memory read and written; the exact step is "
-                "bound by one wave's issue rate on its f64 chains, not by HBM"}
+                "bound by vector issue of its exact products, not by HBM"}
     if with_cpu:
         import orc
         m = orc.Qwen35Model(cfg, tensors, threads=threads)
