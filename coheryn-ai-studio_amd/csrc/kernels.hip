@@ -1932,14 +1932,15 @@ __global__ __launch_bounds__(64 * kQ * kS) void k_mv_f16v(MatrixView w, ActView 
   struct Chunk {
     u32x4v a[kNM], b[kNN];
   };
-  const u32x4v none = {0u, 0u, 0u, 0u};
-  auto load = [&](Chunk &c, int t) {  // inputs past K: zero products
+  // inputs past K: weight +0 and input -0, whose product -0 changes no sum
+  const u32x4v none = {0u, 0u, 0u, 0u}, neg = {0x80008000u, 0x80008000u, 0x80008000u, 0x80008000u};
+  auto load = [&](Chunk &c, int t) {
     const int k = 128 * t + koff;
     const bool in = k < K;
 #pragma unroll
     for (int m = 0; m < kNM; m++) c.a[m] = in ? *reinterpret_cast<const u32x4v *>(wp[m] + k) : none;
 #pragma unroll
-    for (int n = 0; n < kNN; n++) c.b[n] = in ? *reinterpret_cast<const u32x4v *>(xp[n] + k) : none;
+    for (int n = 0; n < kNN; n++) c.b[n] = in ? *reinterpret_cast<const u32x4v *>(xp[n] + k) : neg;
   };
   constexpr int kD = 3;
   Chunk ring[kD];

@@ -37,6 +37,22 @@ def test_f16_matvec_edges(rows, K):
         assert np.array_equal(out.view(np.uint32), sums[..., -1].astype(np.float32).view(np.uint32)), n
 
 
+@pytest.mark.parametrize("K", [32, 96, 128, 160])
+def test_f16_matvec_keeps_the_sign_of_zero(K):
+    """A dot of -0 terms alone is -0, also where K is not whole chunks."""
+    m = host_model()
+    w = np.zeros((9, K), np.float16)
+    w[1] = -0.0
+    for n in (4, 16, 20):
+        print(f"case: f16 zero rows of {K}, {n} inputs", flush=True)
+        x = -np.arange(1, n * K + 1, dtype=np.float32).reshape(n, K) / (n * K)
+        out, _, st, _ = m.matvec(F16, 9, K, w.view(np.uint8), x)
+        assert not st.any()
+        want = np.full((n, 9), 0x80000000, np.uint32)  # +0 weights: -0 products
+        want[:, 1] = 0
+        assert np.array_equal(out.view(np.uint32), want), n
+
+
 @pytest.mark.parametrize("hidden,heads,kv_heads,vocabulary", [(128, 4, 2, 300), (128, 2, 1, 259), (256, 2, 2, 65)])
 @pytest.mark.parametrize("lengths", [(1,), (2, 1, 1), (4, 3, 9), (5, 12, 20), (40, 33, 7)])
 def test_f16_steps_match_oracle(hidden, heads, kv_heads, vocabulary, lengths):
