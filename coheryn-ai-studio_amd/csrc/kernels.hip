@@ -1695,10 +1695,12 @@ __global__ __launch_bounds__(256) void k_mv_f16(MatrixView w, ActView act, int r
 // addition rounded once (the instruction is a chain of four fma).  Every such
 // product is a multiple of 2^-48: a dot whose partial sums stay below 2^5 is
 // exact in f64 in any order, and a larger one rounds at 2^-53 of its size
-// before its final rounding to f32.  The order here is fixed: wave w of the
-// workgroup takes the 32-input blocks w, w + kW, ...; within a block lane
-// group g holds inputs 8g .. 8g+7 (one 16-byte load) and step e multiplies
-// input 8g + e of every group; the waves' sums are added in wave order.
+// before its final rounding to f32.  The order here is the matrix's alone,
+// whatever kNN and kW: the 32-input blocks b fall in classes b % 8, each summed
+// in block order (within a block lane group g holds inputs 8g .. 8g+7, one
+// 16-byte load, and step e multiplies input 8g + e of every group); classes c
+// and c + 4 are added, then the four sums in class order.  Eight waves take a
+// class each, four waves the two classes w and w + 4 in two accumulators.
 //
 // A workgroup owns kNM tiles of 16 output rows x kNN tiles of 16 batch rows.
 // Lane l of an operand tile brings row l % 16 (weights and activations are
@@ -1819,11 +1821,14 @@ __global__ __launch_bounds__(64 * kW) void k_mv_f16m(MatrixView w, ActView act, 
 #pragma unroll
   for (int n = 0; n < kNN; n++)  // rows past the batch repeat its last row
     xp[n] = act.f16 + (size_t)min((ng * kNN + n) * 16 + r16, rows_b - 1) * K + koff;
-  v4d acc[kNM][kNN];
+  constexpr int kA = 8 / kW;  // classes of blocks per wave
+  v4d acc[kA][kNM][kNN];
 #pragma unroll
-  for (int m = 0; m < kNM; m++)
+  for (int c = 0; c < kA; c++)
 #pragma unroll
-    for (int n = 0; n < kNN; n++) acc[m][n] = v4d{-0.0, -0.0, -0.0, -0.0};
+    for (int m = 0; m < kNM; m++)
+#pragma unroll
+      for (int n = 0; n < kNN; n++) acc[c][m][n] = v4d{-0.0, -0.0, -0.0, -0.0};
   struct Block {
     u32x4v a[kNM], b[kNN];
   };
@@ -1834,7 +1839,7 @@ __global__ __launch_bounds__(64 * kW) void k_mv_f16m(MatrixView w, ActView act, 
 #pragma unroll
     for (int n = 0; n < kNN; n++) blk.b[n] = *reinterpret_cast<const u32x4v *>(xp[n] + k);
   };
-  constexpr int kD = 3;
+  constexpr int kD = kA == 1 ? 3 : 4;  // a multiple of kA: slot u holds blocks of class u % kA
   Block ring[kD];
 #pragma unroll
   for (int i = 0; i < kD - 1; i++) load(ring[i], wave + i * kW);
@@ -1855,7 +1860,7 @@ __global__ __launch_bounds__(64 * kW) void k_mv_f16m(MatrixView w, ActView act, 
             const double b = (double)h2f((uint16_t)(blk.b[n][e / 2] >> (16 * (e % 2))));
 #pragma unroll
             for (int m = 0; m < kNM; m++)
-              acc[m][n] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[m], b, acc[m][n], 0, 0, 0);
+              acc[u % kA][m][n] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[m], b, acc[u % kA][m][n], 0, 0, 0);
           }
         }
       }
@@ -1865,10 +1870,13 @@ __global__ __launch_bounds__(64 * kW) void k_mv_f16m(MatrixView w, ActView act, 
 #pragma unroll
   for (int m = 0; m < kNM; m++)
 #pragma unroll
-    for (int n = 0; n < kNN; n++)
+    for (int n = 0; n < kNN; n++) {
+      v4d sum = acc[0][m][n];
+      if constexpr (kA == 2) sum += acc[1][m][n];
 #pragma unroll
       for (int i = 0; i < 4; i++)
-        s_part[(size_t)((wave * kNM + m) * kNN + n) * (16 * kLd) + r16 * kLd + lane / 16 + 4 * i] = acc[m][n][i];
+        s_part[(size_t)((wave * kNM + m) * kNN + n) * (16 * kLd) + r16 * kLd + lane / 16 + 4 * i] = sum[i];
+    }
   __syncthreads();
   // ---- epilogue: thread -> (batch row, output row); 16 consecutive threads
   // hold the 16 outputs of one batch row
@@ -1879,9 +1887,12 @@ __global__ __launch_bounds__(64 * kW) void k_mv_f16m(MatrixView w, ActView act, 
     float v[kNM];
 #pragma unroll
     for (int m = 0; m < kNM; m++) {
-      double sum = s_part[(size_t)(m * kNN + n) * (16 * kLd) + col * kLd + row];
+      double sum = -0.0;
 #pragma unroll
-      for (int i = 1; i < kW; i++) sum += s_part[(size_t)((i * kNM + m) * kNN + n) * (16 * kLd) + col * kLd + row];
+      for (int i = 0; i < 4; i++) {
+        const double *part = s_part + (size_t)((i * kNM + m) * kNN + n) * (16 * kLd) + col * kLd + row;
+        sum += kA == 2 ? part[0] : part[0] + part[(size_t)4 * kNM * kNN * (16 * kLd)];
+      }
       v[m] = (float)sum;
     }
     f16_epilogue<kEpi, kNM>(v, rvalid, r, row0[0] + row, row, w, o, qe, out16, units, unit);
@@ -3191,7 +3202,9 @@ bool launch_gemm_qkv(hipStream_t s, const MatrixView &w, const uint16_t *x, int 
   return true;
 }
 
-// The exact F16 kernels.  Up to 16 rows take k_mv_f16v: at 4 rows down (K
+// The exact F16 kernels.  The forms of k_mv_f16m give the same bits, and so do
+// those of k_mv_f16v for one matrix; the two add in different orders.
+//   Up to 16 rows take k_mv_f16v: at 4 rows down (K
 // 4864) 5.9 us on eight waves per quad, 7.9 on four and 12 on two, sixteen no
 // better; gate+up (1,216 quads) 7.5 on four, 8.9 on eight.  Past 16 rows its
 // smaller tiles lose to k_mv_f16m (56 rows: down 27.4 against 16.4 us, gate+up
