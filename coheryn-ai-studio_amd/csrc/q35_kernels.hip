@@ -229,6 +229,10 @@ __global__ __launch_bounds__(64 * kW) void k_q35_mv(const uint16_t *__restrict__
             for (int r = 0; r < kG; r++) acc[m][g + r] += wd[r];
           }
       }
+      // the sums stay here: sunk past the loop's branch, their terms would
+      // all be live at once (512 registers and scratch where K is ragged)
+#pragma unroll
+      for (int m = 0; m < kTiles; m++) pin_vgprs(acc[m]);
     }
   };
   Step a, b;  // two register sets, one loading while the other is used
