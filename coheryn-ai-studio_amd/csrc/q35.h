@@ -59,8 +59,8 @@ void q35_embed(hipStream_t s, int rows, const uint16_t *embed, const uint32_t *t
 void q35_norm(hipStream_t s, int rows, const float *x, int ldx, const uint32_t *src,
               const float *w, int n, float eps, int zc, float *out, int ldo, uint32_t *row_err,
               const uint32_t *err_row);
-// out[r][o] (=, +=) sum_k f32(x[r][k] * w[o][k]) in f64, in a fixed order;
-// argmax keys per 16-output tile go to part[r][tile] (logits optional).
+// out[r][o] (=, +=) sum_k f32(x[r][k] * w[o][k]) in f64, in an order
+// that K alone fixes; argmax keys per 16-output tile go to part[r][tile] (logits optional).
 void q35_matvec(hipStream_t s, int epi, const uint16_t *w, int rows_w, int valid_rows, int K,
                 const float *x, int ldx, int R, float *out, int ldo, unsigned long long *part,
                 uint32_t *row_err, const uint32_t *err_row);

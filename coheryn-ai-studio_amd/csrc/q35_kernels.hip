@@ -120,35 +120,38 @@ __global__ __launch_bounds__(256) void k_q35_norm(const float *__restrict__ x, i
 // ---------------------------------------------------------------------------
 // BF16 matvec (tensor.rs:380-406 -> cpu::dot): out[r][o] = f32(sum_k
 // f64(f32(w[o][k] * x[r][k]))).  A workgroup owns one tile of 16 outputs x kR
-// rows; its kW waves take 64-input chunks in turn, and within a chunk each
-// 16-lane row of the wave takes 16 inputs: lane l brings the weights of
-// output l % 16 (two 16-byte loads, coalesced in the tile layout).  The rows'
-// inputs pass through a strip of LDS of the wave's own (256 contiguous bytes a
-// row, no barrier: a wave's LDS operations stay in order) and come back as
-// 16-byte broadcasts.  The 4 kW partial sums of an output meet in LDS and are
-// added in a fixed order.  (The reference adds the products in one chain.
-// They are f32 values of 24 bits, so a partial f64 sum rounds only where a
-// product is 2^-29 of it or smaller, by 2^-53 of its size, before the dot is
-// rounded to f32.)
+// rows.  Chunk c of 64 inputs is of class c % 8: eight waves take a class each,
+// four waves the two classes w and w + 4.  Within a chunk each 16-lane row of
+// the wave takes 16 inputs: lane l brings the weights of output l % 16 (two
+// 16-byte loads, coalesced in the tile layout).  The rows' inputs pass through
+// a strip of LDS of the wave's own (256 contiguous bytes a row, no barrier: a
+// wave's LDS operations stay in order) and come back as 16-byte broadcasts.
+//   The order of the sums: a chain per class and 16-lane row, class c + class
+// c + 4, then those by class and row.  It is the same in every instance, so an
+// output does not depend on the rows beside it.  The reference adds the
+// products in one chain; they are f32 values of 24 bits, so a partial f64 sum
+// rounds only where a product is 2^-29 of it or smaller, by 2^-53 of its size,
+// before the dot is rounded to f32.
 //   What bounds it: vector issue, an f32 multiply, a widening and an f64 add
 // per product, 4.6 ns a wave and SIMD, issued as pinned groups of products,
-// widenings and adds over up to eight rows (left alone, the compiler sends
+// widenings and adds over four or eight rows (left alone, the compiler sends
 // every triple through one temporary and each add waits for its widening;
-// taking the inputs from the lanes by DPP, without LDS, cost 5.9 ns).  One chain per output left a decode
-// step waiting on 1,024 to 3,584 dependent adds in every linear.
+// taking the inputs from the lanes by DPP, without LDS, cost 5.9 ns).  One
+// chain per output left a decode step waiting on 1,024 to 3,584 dependent adds
+// in every linear.  Sixteen rows are held to 128 registers, four waves a SIMD
+// (head at 16 rows 330 us; 352 with 154 registers and three waves).
 //   kQ35Swiglu: gate tile blockIdx.x and up tile blockIdx.x + up_off / 16
 // (up_off passed in valid_rows, F in ldo's place as the output count) over the
 // same inputs; h = (g / (1 + exp(-g))) * u (the SwiGLU pass's expression) to
 // out [R][F].
 //   Measured at 16 rows (us a launch, one chain per output before): o 7.3 and
-// down 10.0 (22.4 each), mix 17.1 (22.2), gate+up 15.0 (18.3), head 340 (343);
+// down 10.0 (22.4 each), mix 17.1 (22.2), gate+up 15.0 (18.3), head 330 (343);
 // o and down at 96 rows 28 on average (228).
 // ---------------------------------------------------------------------------
 template <int kEpi, int kR, int kW, bool kTail>
-__global__ __launch_bounds__(64 * kW) void k_q35_mv(const uint16_t *__restrict__ w, int valid_rows, int K,
-                                                    const float *__restrict__ x, int ldx, int R, float *out, int ldo,
-                                                    unsigned long long *__restrict__ part, uint32_t *row_err,
-                                                    const uint32_t *__restrict__ err_row) {
+__global__ __launch_bounds__(64 * kW, kR == 16 && kEpi != kQ35Swiglu && !kTail ? 4 : 1) void k_q35_mv(
+    const uint16_t *__restrict__ w, int valid_rows, int K, const float *__restrict__ x, int ldx, int R, float *out,
+    int ldo, unsigned long long *__restrict__ part, uint32_t *row_err, const uint32_t *__restrict__ err_row) {
   constexpr bool kGlu = kEpi == kQ35Swiglu;
   constexpr int kTiles = kGlu ? 2 : 1;
   __shared__ double s_sum[kW][kTiles][kR][kWave];
@@ -163,11 +166,14 @@ __global__ __launch_bounds__(64 * kW) void k_q35_mv(const uint16_t *__restrict__
   const float *xr[kR];
 #pragma unroll
   for (int r = 0; r < kR; r++) xr[r] = x + (size_t)min(r0 + r, R - 1) * ldx;  // rows past R: unused
-  double acc[kTiles][kR];
+  constexpr int kA = 8 / kW;  // classes of chunks per wave
+  double sums[kA][kTiles][kR];
 #pragma unroll
-  for (int m = 0; m < kTiles; m++)
+  for (int k = 0; k < kA; k++)
 #pragma unroll
-    for (int r = 0; r < kR; r++) acc[m][r] = -0.0;
+    for (int m = 0; m < kTiles; m++)
+#pragma unroll
+      for (int r = 0; r < kR; r++) sums[k][m][r] = -0.0;
   struct Step {
     u32x4q w[kTiles][2];
     float x[kR];
@@ -193,10 +199,10 @@ __global__ __launch_bounds__(64 * kW) void k_q35_mv(const uint16_t *__restrict__
       if (!in) st.x[r] = -0.0f;
     }
   };
-  auto use = [&](const Step &st) {
+  auto use = [&](const Step &st, double (&acc)[kTiles][kR]) {
 #pragma unroll
     for (int r = 0; r < kR; r++) strip[r * kWave + lane] = st.x[r];
-    constexpr int kG = kR < 8 ? kR : 8;
+    constexpr int kG = kR == 8 ? 8 : 4;
 #pragma unroll
     for (int q = 0; q < 4; q++) {  // inputs 4 q .. + 3 of the lane's 16
       float wf[kTiles][4];
@@ -239,28 +245,32 @@ __global__ __launch_bounds__(64 * kW) void k_q35_mv(const uint16_t *__restrict__
   load(a, wave);
   for (int c = wave; c < nc; c += 2 * kW) {
     load(b, c + kW);
-    use(a);
+    use(a, sums[0]);
     if (c + kW < nc) {
       load(a, c + 2 * kW);
-      use(b);
+      use(b, sums[kA - 1]);
     }
   }
   // (each wave's sums take its own strip's place: its reads are behind it)
 #pragma unroll
   for (int m = 0; m < kTiles; m++)
 #pragma unroll
-    for (int r = 0; r < kR; r++) s_sum[wave][m][r][lane] = acc[m][r];
+    for (int r = 0; r < kR; r++)
+      s_sum[wave][m][r][lane] = kA == 1 ? sums[0][m][r] : sums[0][m][r] + sums[kA - 1][m][r];
   __syncthreads();
-  for (int idx = threadIdx.x; idx < kR * 16; idx += 64 * kW) {
+  for (int idx = wave * kWave + (int)__lane_id(); idx < kR * 16; idx += 64 * kW) {
     const int br = idx / 16, oo = idx % 16, r = r0 + br, o = tile * 16 + oo;
     float v[kTiles];
 #pragma unroll
     for (int m = 0; m < kTiles; m++) {
       double sum = -0.0;
 #pragma unroll
-      for (int i = 0; i < kW; i++)
+      for (int i = 0; i < 4; i++)
 #pragma unroll
-        for (int q = 0; q < 4; q++) sum += s_sum[i][m][br][q * 16 + oo];
+        for (int q = 0; q < 4; q++) {
+          const double part = s_sum[i][m][br][q * 16 + oo];
+          sum += kA == 1 ? part + s_sum[i + kW - 4][m][br][q * 16 + oo] : part;
+        }
       v[m] = (float)sum;
     }
     bool bad = !finitef(v[0]);
@@ -1156,7 +1166,7 @@ int q35_matvec_blocks(int rows_w) { return (rows_w + 15) / 16; }
 // down (64 tiles) take 7.3 and 10.0 us as four rows on eight waves, 10.0 and
 // 14.6 as eight; gate+up (224 pairs) 15.0 as eight rows on four waves, 15.2 as
 // four, 18.9 as sixteen; mix (514 tiles) 17.1, 17.2 and 20.1; the head (15,520
-// tiles) 340 as sixteen, 346 as eight, 399 as four.
+// tiles) 330 as sixteen, 346 as eight, 399 as four.  The sums are the same in all.
 template <int kEpi>
 static void mv(hipStream_t s, const uint16_t *w, int tiles, int valid_rows, int K, const float *x, int ldx, int R,
                float *out, int ldo, unsigned long long *part, uint32_t *row_err, const uint32_t *err_row) {
