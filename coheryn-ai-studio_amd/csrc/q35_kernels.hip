@@ -397,14 +397,20 @@ __global__ __launch_bounds__(256) void k_q35_conv(Q35Lanes L, const float *__res
 
 // ---------------------------------------------------------------------------
 // Gated delta rule (kernels.rs:122-214) in three passes.
-// Gates, per (row, value head): the q/k norms (ordered f64 sums of f32
-// squares), q_scale = (1/sqrt(qn + 1e-6))/sqrt(key_dim), k_scale =
+// Gates, per (row, value head): the q/k norms (f64 sums of f32 squares),
+// q_scale = (1/sqrt(qn + 1e-6))/sqrt(key_dim), k_scale =
 // 1/sqrt(kn + 1e-6), decay = exp(log_decay) with log_decay = -exp(A_log) *
 // softplus(a + dt_bias), beta = sigmoid(b) (execution.rs:376-388).
 // ---------------------------------------------------------------------------
-// One wave per (row, value head), the squares added in index order within a
-// lane and over the wave in a fixed tree: 44 us at 4,104 rows x 16 heads, 74
-// with one lane of a workgroup running the whole sum.
+// One wave per (row, value head), the squares added as a tree over the
+// channels, neighbours first (the fused mixer's order): 44 us at 4,104 rows x
+// 16 heads, 74 with one lane of a workgroup running the whole sum.
+template <int kN>  // over aligned groups of kN lanes, the same bits in each lane
+__device__ __forceinline__ double pairs_sum(double v) {
+#pragma unroll
+  for (int m = 1; m < kN; m <<= 1) v += __shfl_xor(v, m, kWave);
+  return v;
+}
 __global__ __launch_bounds__(256) void k_q35_gates(const float *__restrict__ conv, int ldc,
                                                    int keys, const float *__restrict__ mix,
                                                    int ldm, int a_off, int b_off,
@@ -419,16 +425,13 @@ __global__ __launch_bounds__(256) void k_q35_gates(const float *__restrict__ con
   const float *cr = conv + (size_t)row * ldc, *mr = mix + (size_t)row * ldm;
   const float av = mr[a_off + h], bv = mr[b_off + h];
   double q2 = -0.0, k2 = -0.0;
-#pragma unroll
-  for (int c = 0; c < 2; c++) {  // KD <= 128
-    const int i = lane + c * kWave;
-    if (i < KD) {
-      const float q = cr[src + i], k = cr[keys + src + i];
-      q2 += (double)(q * q);
-      k2 += (double)(k * k);
-    }
+  if (2 * lane < KD) {  // KD <= 128; rows and channel offsets are even
+    const float2 q = *reinterpret_cast<const float2 *>(cr + src + 2 * lane);
+    const float2 k = *reinterpret_cast<const float2 *>(cr + keys + src + 2 * lane);
+    q2 = (double)(q.x * q.x) + (double)(q.y * q.y);
+    k2 = (double)(k.x * k.x) + (double)(k.y * k.y);
   }
-  const float qn = (float)wave_sum_f64(q2), kn = (float)wave_sum_f64(k2);
+  const float qn = (float)pairs_sum<kWave>(q2), kn = (float)pairs_sum<kWave>(k2);
   if (lane == 0) {
     const float ld = -exp_f32(a_log[h]) * softplus_f32(av + dt[h]);
     const float beta = sigmoid_f32(bv);
@@ -592,9 +595,10 @@ __global__ __launch_bounds__(256) void k_q35_delta(Q35Lanes L, const float *__re
 // workgroup, token after token (execution.rs:357-411): the causal conv of the
 // head's q, k (its key head's channels) and v channels, the q/k norms and
 // gates, the delta-rule column updates, and the output norm times SiLU(z).
-// kP lanes own one state column, kKD / kP keys each, as in k_q35_delta, and
-// every sum is a fixed tree as in the separate kernels; the arithmetic of each
-// stage is theirs.  (One thread per column with ordered sums took 19 us a
+// kP lanes own one state column, kKD / kP keys each.  The arithmetic of each
+// stage and the order of each sum are the separate kernels' (sums of 16 keys,
+// then a tree over them), so a lane's results do not depend on which of the two
+// runs it.  (One thread per column with ordered sums took 19 us a
 // launch at 16 one-token lanes x 16 heads, most of it waiting on one lane's
 // adds; this takes 15.  Whole waves hold one part of the columns, so the state
 // streams in 256-byte rows and the partial sums meet in LDS: with the lanes of
@@ -642,11 +646,11 @@ __global__ __launch_bounds__(1024) void k_q35_linear(
     const float *__restrict__ a_log, const float *__restrict__ dt,
     const float *__restrict__ norm_w, int KH, int VH, int VD, float eps, float *state,
     size_t state_seq, float *__restrict__ tgt, int ldt, uint32_t *row_err) {
-  constexpr int kCells = kKD / kP;                // keys per thread
+  constexpr int kCells = kKD / kP, kHalves = kCells / 16;  // keys per thread, in sums of 16
   constexpr int kN = kKD < kWave ? kKD : kWave;   // channels of one norm partial
   __shared__ __align__(16) float s_q[kKD], s_k[kKD], s_v[256];
   __shared__ double s_p[2][1024];
-  __shared__ double s_sq[1024 / kN], s_o[1024 / kWave];
+  __shared__ double s_sq[1024 / kN], s_o[256];
   __shared__ float s_decay, s_beta;
   __shared__ int s_bad;
   __shared__ uint64_t s_tab[32];
@@ -690,15 +694,21 @@ __global__ __launch_bounds__(1024) void k_q35_linear(
   const float nw = active ? norm_w[j] : 0.0f;
   __builtin_amdgcn_sched_barrier(0);
   __syncthreads();  // s_tab
-  // a column's partial sums meet in LDS and are added in part order
-  auto all_parts = [&](int which, double v) {
-    if constexpr (kP == 1) return v;
-    s_p[which][tid] = v;
-    __syncthreads();
-    double sum = s_p[which][j];
+  // a column's partial sums meet in LDS and are added in parts_sum's order
+  auto all_parts = [&](int which, const double (&v)[kHalves]) {
+    double p[kP];
+    p[0] = kHalves == 1 ? v[0] : v[0] + v[kHalves - 1];
+    if constexpr (kP > 1) {
+      s_p[which][tid] = p[0];
+      __syncthreads();
 #pragma unroll
-    for (int i = 1; i < kP; i++) sum += s_p[which][i * vdp + j];
-    return sum;
+      for (int i = 0; i < kP; i++) p[i] = s_p[which][i * vdp + j];
+#pragma unroll
+      for (int m = 1; m < kP; m <<= 1)
+#pragma unroll
+        for (int i = 0; i < kP; i += 2 * m) p[i] += p[i + m];
+    }
+    return p[0];
   };
   for (uint32_t t = 0; t < n; t++) {
     const uint32_t row = first + t;
@@ -717,9 +727,7 @@ __global__ __launch_bounds__(1024) void k_q35_linear(
       }
     }
     // q/k norms: a tree over each kN channels, then (128 keys) two in order
-    double sq = (double)(y * y);
-#pragma unroll
-    for (int m = 1; m < kN; m <<= 1) sq += __shfl_xor(sq, m, kWave);
+    const double sq = pairs_sum<kN>((double)(y * y));
     if (tid % kN == 0) s_sq[tid / kN] = sq;
     if (gate) {
       const float ld = -exp_f32_tab(al, s_tab) * softplus_f32(a_in + dtb, s_tab);
@@ -743,7 +751,7 @@ __global__ __launch_bounds__(1024) void k_q35_linear(
     float o = 0.0f;
     {
       const float decay = s_decay, beta = s_beta, v = s_v[min(j, VD - 1)];
-      double pred = 0.0;
+      double pred[kHalves] = {};
       float kk[kCells];
 #pragma unroll
       for (int u = 0; u < kCells / 4; u++) {
@@ -754,10 +762,10 @@ __global__ __launch_bounds__(1024) void k_q35_linear(
 #pragma unroll
       for (int i = 0; i < kCells; i++) {
         col[i] *= decay;
-        pred += (double)(col[i] * kk[i]);
+        pred[i / 16] += (double)(col[i] * kk[i]);
       }
       const float corr = (v - (float)all_parts(0, pred)) * beta;
-      double rd = 0.0;
+      double rd[kHalves] = {};
 #pragma unroll
       for (int u = 0; u < kCells / 4; u++) {
         const float4 a = *reinterpret_cast<const float4 *>(&s_q[part % kP * kCells + 4 * u]);
@@ -765,7 +773,7 @@ __global__ __launch_bounds__(1024) void k_q35_linear(
 #pragma unroll
         for (int e = 0; e < 4; e++) {
           col[4 * u + e] += kk[4 * u + e] * corr;
-          rd += (double)(col[4 * u + e] * qq[e]);
+          rd[u / 4] += (double)(col[4 * u + e] * qq[e]);
         }
       }
       // a non-finite updated cell makes o non-finite (its read product is
@@ -774,12 +782,16 @@ __global__ __launch_bounds__(1024) void k_q35_linear(
       bad |= active && !finitef(o);
     }
     // output norm over the head (zero_centered false) times SiLU(z) (execution.rs:397-411)
-    const double os = wave_sum_f64(active && part == 0 ? (double)(o * o) : -0.0);
-    if (tid % kWave == 0) s_o[tid / kWave] = os;
+    // its sum as in k_q35_headnorm, by every wave
+    if (active && part == 0) s_o[j] = (double)(o * o);
     __syncthreads();
-    double sum = s_o[0];
-    for (int i = 1; i < (int)blockDim.x / kWave; i++) sum += s_o[i];
-    const double mean = sum / (double)VD;
+    double os = -0.0;
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+      const int i = tid % kWave + c * kWave;
+      if (i < VD) os += s_o[i];
+    }
+    const double mean = wave_sum_f64(os) / (double)VD;
     bad |= !(__builtin_isfinite(mean) && finitef((float)mean));
     if (active && part == 0) {
       const float yo = ((o * (1.0f / sqrtf((float)mean + eps))) * (nw + 0.0f)) * silu_f32(z, s_tab);

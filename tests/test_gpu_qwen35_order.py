@@ -97,3 +97,39 @@ def test_hybrid_linears_do_not_depend_on_the_batch():
                 name.endswith(("q_proj.weight", "k_proj.weight", "v_proj.weight")):
             edit(t, name, cancel)
     assert schedules(cfg, t, LENGTHS, 3) == 0
+
+
+@pytest.mark.parametrize("key_dim,value_dim", [(32, 40), (64, 64), (128, 128), (128, 200)])
+def test_hybrid_mixer_does_not_depend_on_the_chunking(key_dim, value_dim):
+    """Chunks of five tokens and more run the mixer's separate kernels, one
+    token the fused one.  Query channels a and b of a head are negated copies
+    (their taps are small enough that SiLU halves them exactly) and the key
+    channels equal ones, so cells a and b cancel in the head's read sum."""
+    print(f"case: hybrid mixer, chunks against single tokens, {key_dim} keys x {value_dim}", flush=True)
+    heads = 2
+    cfg = tiny(layers=2, pattern="LF", hidden=128, vocabulary=300, key_heads=heads, value_heads=heads,
+               key_dim=key_dim, value_dim=value_dim)
+    cfg, t = synth35.in_memory(cfg, seed=key_dim + value_dim)
+    keys = heads * key_dim
+    rng = np.random.default_rng(key_dim)
+    pairs = [(h * key_dim + a, h * key_dim + b) for h in range(heads)
+             for a, b in rng.permutation(key_dim)[:key_dim // 4 * 2].reshape(-1, 2)]
+    pa, pb = (np.array(v) for v in zip(*pairs))
+    lone = np.setdiff1d(np.arange(keys), np.concatenate([pa, pb]))
+    p = "model.language_model.layers.0.linear_attn"
+
+    def rows(f):
+        f[pb], f[keys + pb] = f[pa], f[keys + pa]
+        return f
+
+    def taps(f):
+        f = f.reshape(-1, cfg["conv_kernel"])
+        f[:keys] *= 2.0 ** -28
+        f[pb], f[keys + pb] = -f[pa], f[keys + pa]
+        f[lone] *= 2.0 ** -32
+        return f.reshape(-1)
+
+    edit(t, f"{p}.in_proj_qkv.weight", rows)
+    edit(t, f"{p}.conv1d.weight", taps)
+    edit(t, f"{p}.out_proj.weight", lambda f: f * 2.0 ** 50)
+    assert schedules(cfg, t, (9, 5, 12, 7), 3) == 0
