@@ -251,7 +251,9 @@ __global__ __launch_bounds__(64 * kW, kR == 16 && kEpi != kQ35Swiglu && !kTail ?
       use(b, sums[kA - 1]);
     }
   }
-  // (each wave's sums take its own strip's place: its reads are behind it)
+  // each wave's sums take its own strip's place; the fence keeps its reads of
+  // the strip (another type, which the compiler need not order) ahead of them
+  asm volatile("" ::: "memory");
 #pragma unroll
   for (int m = 0; m < kTiles; m++)
 #pragma unroll
