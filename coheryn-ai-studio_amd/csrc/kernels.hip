@@ -2761,7 +2761,7 @@ __global__ __launch_bounds__(64 * kG) void k_attn_chunk(StepDims d, const int4 *
 
 // Pass 4: chunks combined in order, rounded to f32, and prepared as the
 // operand of attn_output (each head's D elements hold whole Q8_0 blocks).
-// kWide: blockDim.y heads per workgroup, each on whole waves; else one head,
+// kWide (F16 rows): blockDim.y heads per workgroup, each on whole waves; else one head,
 // with nothing ahead of the first load that depends on the block's shape
 // (heads taken from the thread id by division cost decode steps about 0.5%).
 template <int kAct, bool kWide>
@@ -2769,13 +2769,13 @@ __global__ __launch_bounds__(kWide ? 256 : 128) void k_attn_combine(StepDims d,
                                                                     const uint32_t *__restrict__ row_pos,
                                                                     const double *__restrict__ partial, int nbp,
                                                                     ActView act, uint32_t *row_err) {
-  __shared__ float s_o[kWide ? 256 : 128];
+  static_assert(!kWide || kAct == kActF16, "the quantized forms share o_s within a head");
+  __shared__ float o_s[128];
   const int sub = kWide ? __builtin_amdgcn_readfirstlane(threadIdx.y) : 0;
   const int r = blockIdx.x, j = threadIdx.x, h = kWide ? blockIdx.y * blockDim.y + sub : blockIdx.y;
-  float *o_s = s_o + (kWide ? sub * blockDim.x : 0);
   const int kv = (int)row_pos[r] + 1, nch = (kv + kChunk - 1) / kChunk;
   const double *pp = partial + ((size_t)r * d.NH + h) * d.max_chunks * d.D;
-  const bool live = !kWide || h < d.NH, active = live && j < d.D;
+  const bool active = (!kWide || h < d.NH) && j < d.D;
   double acc = 0.0;
   const bool direct = d.row_skip && d.row_skip[r];
   if (active && !direct) {
@@ -2837,7 +2837,7 @@ __global__ __launch_bounds__(kWide ? 256 : 128) void k_attn_combine(StepDims d,
     float v[8];
 #pragma unroll
     for (int i = 0; i < 8; i++) v[i] = j < ng ? o_s[j * 8 + i] : 0.0f;
-    if (live && j < ((ng + 3) & ~3))
+    if (j < ((ng + 3) & ~3))
       bad |= quant_group_q8<1, kAct == kActQ8H>(v, j < ng, r, h * ng + j, nbp, act);
   } else if (kAct == kActF32) {  // f32 rows for a following Q8_K quantizer
     if (active) act.f32[(size_t)r * d.H + h * d.D + j] = o;
@@ -3516,28 +3516,25 @@ void launch_attn_chunk(hipStream_t s, int n_tiles, const StepDims &d, const int4
 void launch_attn_combine(hipStream_t s, int rows, const StepDims &d, const uint32_t *row_pos,
                          const double *partial, int act_dtype, int nbp, ActView act,
                          uint32_t *row_err) {
-  // a workgroup of one head, or of 256 threads' heads where (row, head)
-  // workgroups number in the ten thousands and their dispatch sets the pace
-  // (2,616 rows x 14 heads: 19.4 -> 17.0 us)
+  // a workgroup of one head, or for F16 rows of 256 threads' heads where (row,
+  // head) workgroups number in the ten thousands and their dispatch sets the
+  // pace (2,616 rows x 14 heads: 19.9 -> 15.3 us).  The quantized forms gain
+  // nothing there (23.5 against 23.8 us): eight lanes of a head's wave quantize
+  // after the others.
   const int tph = ((d.D + kWave - 1) / kWave) * kWave;
-  const bool wide = rows * d.NH >= 8192;
+  const bool wide = act_dtype == kActF16 && rows * d.NH >= 8192;
   const int heads = wide ? 256 / tph : 1;
   const dim3 grid(rows, (d.NH + heads - 1) / heads), block(tph, heads);
-  auto go = [&](auto kact) {
-    constexpr int kAct = decltype(kact)::value;
-    if (wide)
-      launch_k((k_attn_combine<kAct, true>), grid, block, 0, s, d, row_pos, partial, nbp, act, row_err);
-    else
-      launch_k((k_attn_combine<kAct, false>), grid, block, 0, s, d, row_pos, partial, nbp, act, row_err);
-  };
-  if (act_dtype == kActQ8)
-    go(std::integral_constant<int, kActQ8>());
+  if (wide)
+    launch_k((k_attn_combine<kActF16, true>), grid, block, 0, s, d, row_pos, partial, nbp, act, row_err);
+  else if (act_dtype == kActQ8)
+    launch_k((k_attn_combine<kActQ8, false>), grid, block, 0, s, d, row_pos, partial, nbp, act, row_err);
   else if (act_dtype == kActQ8H)
-    go(std::integral_constant<int, kActQ8H>());
+    launch_k((k_attn_combine<kActQ8H, false>), grid, block, 0, s, d, row_pos, partial, nbp, act, row_err);
   else if (act_dtype == kActF32)
-    go(std::integral_constant<int, kActF32>());
+    launch_k((k_attn_combine<kActF32, false>), grid, block, 0, s, d, row_pos, partial, nbp, act, row_err);
   else
-    go(std::integral_constant<int, 1>());
+    launch_k((k_attn_combine<kActF16, false>), grid, block, 0, s, d, row_pos, partial, nbp, act, row_err);
 }
 
 void launch_fill_synthetic(hipStream_t s, float *kpool, float *vpool, size_t layer_stride,
