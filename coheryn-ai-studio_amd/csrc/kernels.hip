@@ -735,12 +735,14 @@ __device__ __forceinline__ void kq_split(uint2 q, uint32_t sc, long &hi, long &l
   lo = (long)(((unsigned long)l[1] << 32) | l[0]);
 }
 
-// The loads of a block run two blocks ahead of their use (each block used to
-// wait for its own: down at 32 rows 19.5 us, 11.4 now), and a workgroup takes
-// kNN batch tiles, which share each weight's scaling and split.
-template <int kEpi, int kNM, int kNN>
-__global__ __launch_bounds__(512) void k_mv_kq(MatrixView w, ActView act, int rows_b, int n_tiles,
-                                               MatvecOut o) {
+// kD blocks are in flight: three where few workgroups leave a CU waiting (down
+// at 32 rows 19.5 us with one, 11.4 with three), one where four of them (57
+// registers) cover each other.  A workgroup takes kNN batch tiles, which share
+// each weight's scaling and split.
+template <int kEpi, int kNM, int kNN, int kD>
+__global__ __launch_bounds__(512, kD == 1 && kNN * kNM == 1 ? 8 : 1) void k_mv_kq(MatrixView w, ActView act,
+                                                                                 int rows_b, int n_tiles,
+                                                                                 MatvecOut o) {
   __shared__ float s_lane[8][kNM * kNN][256];
   __shared__ float s_min[kNM * kNN][256];
   __shared__ unsigned long long s_key[kNN][4][16];
@@ -847,7 +849,6 @@ __global__ __launch_bounds__(512) void k_mv_kq(MatrixView w, ActView act, int ro
       }
     }
   };
-  constexpr int kD = 3;
   Block ring[kD];
 #pragma unroll
   for (int i = 0; i < kD - 1; i++) load(ring[i], i);
@@ -3293,20 +3294,34 @@ bool launch_matvec_swiglu_f16(hipStream_t s, const MatrixView &w, const ActView 
 template <int kEpi, int kNM>
 static void mv_kq(hipStream_t s, const MatrixView &w, const ActView &act, int rows_b, const MatvecOut &o) {
   const int units = w.mtiles / kNM, n_tiles = (rows_b + 15) / 16;
-  auto go = [&](auto nn) {
-    constexpr int kNN = decltype(nn)::value;
+  auto go = [&](auto nn, auto d) {
+    constexpr int kNN = decltype(nn)::value, kD = decltype(d)::value;
     const int groups = (n_tiles + kNN - 1) / kNN;
-    launch_k((k_mv_kq<kEpi, kNM, kNN>), dim3((units + 7) / 8 * 8 * groups), dim3(512), 0, s, w, act, rows_b, n_tiles,
-             o);
+    launch_k((k_mv_kq<kEpi, kNM, kNN, kD>), dim3((units + 7) / 8 * 8 * groups), dim3(512), 0, s, w, act, rows_b,
+             n_tiles, o);
   };
-  // one batch tile per workgroup keeps the grid wide at few rows (down at 32
-  // rows: 11.4 us, 16.1 as two, 19.9 as three); from eight tiles on the shared
-  // loads and splits win (387 rows: 50.9 as one, 41.9 as two, 37.4 as three;
-  // three tiles of a gate and up pair would leave one wave a SIMD)
-  if (n_tiles >= 8)
-    go(std::integral_constant<int, kNM == 2 ? 2 : 3>{});
+  // rounds of one workgroup per CU; several resident ones share its time
+  auto rounds = [&](int nn) { return (units * ((n_tiles + nn - 1) / nn) + 255) / 256; };
+  using std::integral_constant;
+  // One round waits on memory: three blocks in flight (2,048 x 6,144 at 16
+  // rows, Q4_K: 16.8 us, 19.5 with one; at K = 1,024 they are the whole row).
+  // More rounds cover each other's waits with small workgroups, and the ring
+  // costs more than it hides (50,000 x 1,024 at 16 rows 53.7 us, 31.5 with one
+  // block in flight).  A round of two batch tiles takes 1.6 rounds of one (at
+  // 32 rows 97 as one, 47.5 as two; at 48 rows 79.7 as one, 84.5 as two).
+  // Three, in flight, take 2.2: they win where their rounds are one or two
+  // deep ones and fit better (2,048 x 6,144 at 80 rows: 29.6 us, 41.6 as one,
+  // 41.2 as two; 32,000 x 4,096 at 80 rows 327, 309, 281).
+  const int one = rounds(1) * 100, two = rounds(2) * 160, three = rounds(3) * 220;
+  if constexpr (kNM == 1) {
+    if (rounds(1) == 1 && w.nb >= 6) return go(integral_constant<int, 1>{}, integral_constant<int, 3>{});
+    if (rounds(3) <= 2 && w.nb >= 16 && three < one && three < two)
+      return go(integral_constant<int, 3>{}, integral_constant<int, 3>{});
+  }
+  if (one <= two)
+    go(integral_constant<int, 1>{}, integral_constant<int, 1>{});
   else
-    go(std::integral_constant<int, 1>{});
+    go(integral_constant<int, 2>{}, integral_constant<int, 1>{});
 }
 
 bool launch_matvec(hipStream_t s, Epilogue epi, const MatrixView &w, const ActView &act,

@@ -80,16 +80,22 @@ def test_f16_combine_of_several_heads(hidden, heads, kv_heads):
     check(c, m, o, [((rows + lanes - 1) // lanes,) * lanes], 256)
 
 
-def test_kquant_wide_steps():
-    """All matrices K-quants: 130 prompt rows (gate+up in pairs of batch tiles)
-    and 130 and 113 decoding lanes (the head in threes)."""
-    print("case: K-quant steps of 130 rows and 130 lanes", flush=True)
-    cfg = synth.config(layers=2, hidden=256, intermediate=512, heads=4, kv_heads=2, vocabulary=300, context=256)
+@pytest.mark.parametrize("hidden,intermediate,heads,plan", [
+    (1024, 4096, 16, ((9,), (20,), (30, 40), (10, 33, 50, 37), (1,) * 70, (1,) * 130)),
+    (4096, 256, 64, ((1,) * 20, (1,) * 130))])
+def test_kquant_wide_steps(hidden, intermediate, heads, plan):
+    """All matrices K-quants, prompt and decode steps of 9 to 130 rows: 64
+    output tiles with a long K (down at 1,024, the head at 4,096) and a short
+    one, and 256 gate and up pairs, which take one, two and three batch tiles a
+    workgroup."""
+    print(f"case: K-quant steps, hidden {hidden}", flush=True)
+    cfg = synth.config(layers=1, hidden=hidden, intermediate=intermediate, heads=heads, kv_heads=heads // 8,
+                       vocabulary=1011, context=256)
     c, t = synth.in_memory(cfg, "q4_k_m", seed=11)
     print("dtypes:", model_dtypes(t), flush=True)
-    m = cohx.Model(c, t, max_lanes=130, max_rows=130, max_seqs=130, max_context=64)
+    m = cohx.Model(c, t, max_lanes=130, max_rows=130, max_seqs=130, max_context=128)
     o = orc.Model(c, t, threads=8)
-    check(c, m, o, [(40, 33, 20, 37), (1,) * 130, (1,) * 113], 64)
+    check(c, m, o, plan, 128)
 
 
 @pytest.mark.parametrize("hidden", [64, 72])
