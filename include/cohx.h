@@ -287,7 +287,9 @@ typedef struct {
  *     as ne0 = K, ne1 = C;
  *   cohx_finalize; cohx_seq_alloc / free / length;
  *   cohx_seq_fork: a full snapshot copy at the source's length (recurrent state
- *     cannot be shared; execution.rs:117-133);
+ *     cannot be shared; execution.rs:117-133).  It returns once the copy is
+ *     queued: steps and reads that follow see the whole copy, and a device
+ *     error of the copy is reported by the next call that waits for the device;
  *   cohx_seq_read_kv: values 0/1 = K/V rows [0, length) of a full-attention
  *     layer, 2 = conv ring [channels][kernel], 3 = delta memory
  *     [value_heads][key_dim][value_dim] of a linear-attention layer;
