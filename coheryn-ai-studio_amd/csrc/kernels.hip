@@ -7,8 +7,8 @@
 //    reference's per-block chain sum = fmaf(float(isum), dw*da, sum) in block
 //    order for every (row, lane) — quant.rs:265-272.
 //  * attention scores: q.k summed in f64 in element order, as cpu.rs:31-35.
-//  * f64 sums over many elements (RMSNorm, softmax denominator, P.V) use a
-//    fixed tree / chunk order; they equal the sequential sum whenever no
+//  * f64 sums over many elements (RMSNorm, softmax denominator, P.V, the F16
+//    dot) use a fixed tree / chunk order; they equal the sequential sum whenever no
 //    partial sum rounds, and otherwise differ below 2^-52 relative before the
 //    final rounding to f32.
 #include <hip/hip_ext.h>
@@ -1727,65 +1727,65 @@ __device__ __forceinline__ void f16_epilogue(const float (&v)[kNM], bool rvalid,
                                              uint16_t *out16, int tiles, int tile) {
   bool bad = false;
   const int F = w.rows / 2;
-      if constexpr (kEpi == kEpiArgmax) {
-        const bool valid = rvalid && orow < w.rows;
-        if (valid) {
-          bad = !finitef(v[0]);
-          if (o.logits) o.logits[(size_t)r * w.rows + orow] = v[0];
-        }
-        unsigned long long key = valid ? argmax_key(v[0], orow) : 0ull;
+  if constexpr (kEpi == kEpiArgmax) {
+    const bool valid = rvalid && orow < w.rows;
+    if (valid) {
+      bad = !finitef(v[0]);
+      if (o.logits) o.logits[(size_t)r * w.rows + orow] = v[0];
+    }
+    unsigned long long key = valid ? argmax_key(v[0], orow) : 0ull;
 #pragma unroll
-        for (int s = 1; s < 16; s <<= 1) {
-          const unsigned long long x = __shfl_xor(key, s, kWave);
-          key = x > key ? x : key;
+    for (int s = 1; s < 16; s <<= 1) {
+      const unsigned long long x = __shfl_xor(key, s, kWave);
+      key = x > key ? x : key;
+    }
+    if (rvalid && row == 0) o.argmax[(size_t)r * tiles + tile] = key;
+  } else if constexpr (kEpi == kEpiQkv) {
+    // k_qkv_post's arithmetic: element i of a head in v[0], i + D/2 in v[1]
+    if (rvalid) {
+      bad = !finitef(v[0]) || !finitef(v[kNM - 1]);
+      const uint32_t pos = qe.row_pos[r];
+      const int32_t slot = qe.row_slot[r];
+      const int half = qe.D / 2, page = slot / kPage, off = slot % kPage;
+      const int head = orow / qe.D, i = orow % qe.D;
+      const float a = v[0] + qe.bias[orow], b = v[kNM - 1] + qe.bias[orow + half];
+      const int nh = qe.H / qe.D;
+      if (head < nh + qe.NKV) {
+        const float2 cs = qe.rope[(size_t)pos * half + i];
+        const float ya = fmaf(a, cs.x, -(b * cs.y)), yb = fmaf(a, cs.y, b * cs.x);
+        if (head < nh) {
+          float *q = qe.q_rot + (size_t)r * qe.H + orow;
+          q[0] = ya;
+          q[half] = yb;
+        } else if (slot >= 0) {
+          qe.kpool[k_at(page, pos / kPage, head - nh, qe.NKV, off, i, qe.D)] = ya;
+          qe.kpool[k_at(page, pos / kPage, head - nh, qe.NKV, off, i + half, qe.D)] = yb;
         }
-        if (rvalid && row == 0) o.argmax[(size_t)r * tiles + tile] = key;
-      } else if constexpr (kEpi == kEpiQkv) {
-        // k_qkv_post's arithmetic: element i of a head in v[0], i + D/2 in v[1]
-        if (rvalid) {
-          bad = !finitef(v[0]) || !finitef(v[kNM - 1]);
-          const uint32_t pos = qe.row_pos[r];
-          const int32_t slot = qe.row_slot[r];
-          const int half = qe.D / 2, page = slot / kPage, off = slot % kPage;
-          const int head = orow / qe.D, i = orow % qe.D;
-          const float a = v[0] + qe.bias[orow], b = v[kNM - 1] + qe.bias[orow + half];
-          const int nh = qe.H / qe.D;
-          if (head < nh + qe.NKV) {
-            const float2 cs = qe.rope[(size_t)pos * half + i];
-            const float ya = fmaf(a, cs.x, -(b * cs.y)), yb = fmaf(a, cs.y, b * cs.x);
-            if (head < nh) {
-              float *q = qe.q_rot + (size_t)r * qe.H + orow;
-              q[0] = ya;
-              q[half] = yb;
-            } else if (slot >= 0) {
-              qe.kpool[k_at(page, pos / kPage, head - nh, qe.NKV, off, i, qe.D)] = ya;
-              qe.kpool[k_at(page, pos / kPage, head - nh, qe.NKV, off, i + half, qe.D)] = yb;
-            }
-          } else if (slot >= 0) {
-            qe.vpool[v_at(page, head - nh - qe.NKV, qe.NKV, off, i, qe.D)] = a;
-            qe.vpool[v_at(page, head - nh - qe.NKV, qe.NKV, off, i + half, qe.D)] = b;
-          }
-        }
-      } else if (rvalid) {
-        if constexpr (kEpi == kEpiSwiglu) {
-          if (orow < F) {
-            const float g = v[0], u = v[kNM - 1];
-            bad = !finitef(g) || !finitef(u);
-            const float y = (g / (1.0f + exp_f32(-g))) * u;
-            if (out16) {  // k_quant_act<1>'s rounding and check
-              const uint16_t h = f2h(y);
-              bad |= !finitef(h2f(h));
-              out16[(size_t)r * F + orow] = h;
-            } else {
-              o.out[(size_t)r * o.ld + orow] = y;
-            }
-          }
-        } else if (orow < w.rows) {
-          bad = !finitef(v[0]);
-          float *p = o.out + (size_t)r * o.ld + orow;
-          *p = kEpi == kEpiResidual ? *p + v[0] : v[0];
+      } else if (slot >= 0) {
+        qe.vpool[v_at(page, head - nh - qe.NKV, qe.NKV, off, i, qe.D)] = a;
+        qe.vpool[v_at(page, head - nh - qe.NKV, qe.NKV, off, i + half, qe.D)] = b;
+      }
+    }
+  } else if (rvalid) {
+    if constexpr (kEpi == kEpiSwiglu) {
+      if (orow < F) {
+        const float g = v[0], u = v[kNM - 1];
+        bad = !finitef(g) || !finitef(u);
+        const float y = (g / (1.0f + exp_f32(-g))) * u;
+        if (out16) {  // k_quant_act<1>'s rounding and check
+          const uint16_t h = f2h(y);
+          bad |= !finitef(h2f(h));
+          out16[(size_t)r * F + orow] = h;
+        } else {
+          o.out[(size_t)r * o.ld + orow] = y;
         }
       }
+    } else if (orow < w.rows) {
+      bad = !finitef(v[0]);
+      float *p = o.out + (size_t)r * o.ld + orow;
+      *p = kEpi == kEpiResidual ? *p + v[0] : v[0];
+    }
+  }
   if (bad) atomicOr(&o.row_err[o.err_rows ? (int)o.err_rows[r] : r], kErrNonFinite);
 }
 

@@ -506,7 +506,8 @@ int q35_read_state(cohx_ctx *ctx, uint32_t seq, uint32_t layer, int which, float
 // Graph::forward_batch over a ragged batch (execution.rs:257-608): a lane may
 // carry several consecutive tokens (a prompt chunk); the linears run over all
 // packed rows, and the recurrences walk each lane's tokens in order, so the
-// result equals stepping the tokens one at a time.
+// result equals stepping the tokens one at a time (bit for bit on the exact
+// kernels, whose sums do not depend on the batch).
 int q35_step(cohx_ctx *ctx, const cohx_batch *batch, cohx_step_out *out, const cohx_step_hooks *hooks) {
   const auto t_start = std::chrono::steady_clock::now();
   Q35Model *q = ctx->q35;

@@ -1,8 +1,14 @@
-// Qwen3.5 hybrid text step on the GPU, exact: every kernel reproduces the
-// engine's float arithmetic (crates/coheryn-engine/src/qwen35/execution.rs:
-// 257-608, qwen35/kernels.rs:11-269, cpu.rs:31-35,74-124) bit for bit:
-// f32 products, f64 sums in the reference's element order, glibc expf and
-// log1pf restated (exp_f32, log1p_f32), no contraction.
+// Qwen3.5 hybrid text step on the GPU: the engine's float arithmetic
+// (crates/coheryn-engine/src/qwen35/execution.rs:257-608, qwen35/kernels.rs:
+// 11-269, cpu.rs:31-35,74-124): its f32 products, glibc expf and log1pf
+// restated (exp_f32, log1p_f32), no contraction.  The conv, the attention
+// scores and the softmax recurrences run in the reference's element order.  The
+// f64 sums of the linears, the norms, the gates' q/k squares and the delta rule
+// are split over lanes and waves where the reference runs one chain: the same
+// bits unless a partial sum rounds in f64 and the difference crosses an f32
+// rounding boundary.  Their orders are fixed by the model's shape, so a lane's
+// results depend neither on the rows and lanes beside it nor on how its tokens
+// are cut into steps.
 //
 // Layout: activations are row-major f32 per packed row; matrices are BF16
 // tiles of 16 outputs (q35_tiled_index); the sequence state lives in slabs

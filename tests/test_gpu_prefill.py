@@ -314,7 +314,7 @@ def test_regime_head_on_matrix_cores_matches_oracle():
 
 def test_wide_f16_decode_step_stays_exact():
     """A decode-only F16 step of 130 rows, as wide as the regime's steps,
-    keeps the exact kernels (one f64 chain per dot, the exact head): every
+    keeps the exact kernels (f64 sums of the exact products, the exact head): every
     lane's logits and greedy id equal the oracle's bit for bit, with the
     regime switched on."""
     print("case: F16 decode-only step of 130 lanes with the regime on: exact", flush=True)

@@ -2,7 +2,7 @@
 
 Four f64 sums of the exact path run in a fixed order that differs from the
 reference's sequential loops (the rms_norm sum of squares, the softmax
-denominator, the attention value sums, and the F16 dot under 16 rows).  Each
+denominator, the attention value sums, and the F16 dot).  Each
 sums f32 values in f64, so the two orders can differ only in the last f64
 bits, and then only when a partial sum rounds, which needs terms that span
 more than ~29 binades; the f32 result then differs only when the f64 value
