@@ -1706,7 +1706,7 @@ __global__ __launch_bounds__(256) void k_mv_f16(MatrixView w, ActView act, int r
 // A workgroup owns kNM tiles of 16 output rows x kNN tiles of 16 batch rows.
 // Lane l of an operand tile brings row l % 16 (weights and activations are
 // row-major, so a wave's load of a tile is 16 rows x 64 bytes), the loads run
-// two blocks ahead of their use.  What bounds it is the f64 matrix rate: 31 ns
+// one or two blocks ahead of their use.  What bounds it is the f64 matrix rate: 31 ns
 // per instruction and SIMD (1,024 products), against about 75 ns for the same
 // products as f32 multiply, widening and f64 add on the vector unit.
 // kEpiSwiglu pairs gate tile u with up tile u (row + F), kEpiQkv the two tiles
@@ -1840,7 +1840,10 @@ __global__ __launch_bounds__(64 * kW) void k_mv_f16m(MatrixView w, ActView act, 
 #pragma unroll
     for (int n = 0; n < kNN; n++) blk.b[n] = *reinterpret_cast<const u32x4v *>(xp[n] + k);
   };
-  constexpr int kD = kA == 1 ? 3 : 4;  // a multiple of kA: slot u holds blocks of class u % kA
+  // a multiple of kA: slot u holds blocks of class u % kA.  Two accumulators
+  // leave room for one block ahead, not three (gate+up at 56 rows 24.9 us on
+  // 72 registers, 26.4 on 105)
+  constexpr int kD = kA == 1 ? 3 : 2;
   Block ring[kD];
 #pragma unroll
   for (int i = 0; i < kD - 1; i++) load(ring[i], wave + i * kW);
