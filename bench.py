@@ -39,7 +39,7 @@ TRAFFIC_FILE = os.path.join(ROOT, "profiles", "traffic_decode128.json")
 # (qkv, o and down are split-K instances; o and down share one instance and
 # grid, so counters cannot tell them apart)
 CATEGORY_KERNEL = {"attn_scores": "k_attn_scores<64, 7, 2>", "attn_softmax_stats": "k_attn_exp<7>",
-                   "attn_pv": "k_attn_pv<64, 7>", "attn_combine_act": "k_attn_combine<8>",
+                   "attn_pv": "k_attn_pv<64, 7>", "attn_combine_act": "k_attn_combine<8, false>",
                    "matvec_qkv": "k_mv_q8s<4, 1, 2, 8, 8>", "matvec_o_residual": "k_mv_q8s<1, 1, 2, 8, 8>",
                    "matvec_gate_up_swiglu": "k_mv_q8w<2, 2, 8, 14, 2, true>",
                    "matvec_down_residual": "k_mv_q8s<1, 1, 2, 8, 8>",
